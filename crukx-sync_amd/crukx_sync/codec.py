@@ -28,8 +28,8 @@ _MASK64 = (1 << 64) - 1
 # The reference's knob (codec.py:30), with its default: tensors of more than _SLAB elements get their
 # group sizes checked against the receiver's exponent counts before decoding ("group has more changes
 # than elements", codec.py:598-604).  The reference also sorts at most _SLAB elements at once; here one
-# wavefront ranks min(_SLAB, 65536) elements (rounded down to a multiple of 128), and the per-slab
-# exponent histograms are scanned afterwards.  It never changes the bytes.
+# wavefront ranks at most min(_SLAB, 65536) elements (rounded down to a multiple of 128; fewer in small
+# calls), and the per-slab exponent histograms are scanned afterwards.  It never changes the bytes.
 _SLAB = 1 << 24
 
 
@@ -351,9 +351,10 @@ def _encode_call(names, A, B, numels, pa, pb, has, vals, dev):
 _COUNT_CACHE = True
 
 # Receiver-side exponent counts per slab, kept on the device across updates of the same tensors:
-# id(tensor) -> (weakref, _version after our last write, device buffer, slab size, device, buffer
-# address).  They are used only with the same slab size and a checksum-cache hit for the tensor (the
-# same trust rule), and let apply skip its full read of those weights (crx_apply_cached).
+# id(tensor) -> (weakref, _version after our last write, device buffer, _SLAB, device, buffer address,
+# slab size of the counts).  They are used only with the same _SLAB, in an apply that ranks slabs of that
+# size, and with a checksum-cache hit for the tensor (the same trust rule), and let apply skip its full
+# read of those weights (crx_apply_counts).
 _hist = {}
 # Guards _hist across threads.  Reentrant: a weakref callback that drops an entry can run inside a
 # locked region when a garbage collection happens there.
@@ -402,12 +403,28 @@ def _apply_inputs(names, numels, weights, checksums):
             array("Q", [h[0] & _MASK64 if o else 0 for h, o in zip(hits, ok)]), ptrs)
 
 
-def _hist_store(t, buf, slab, dev):
+def _count_slab(u, usable, numels, slab):
+    """The slab size of an apply of `u` to tensors of `numels` elements, whose usable counts are `usable`
+    (an entry of _hist, or None, per tensor): that of the counts that cover half of the elements, so that
+    a receiver whose updates hold now more, now fewer of its tensors or changes keeps its counts; else the
+    one that suits the update."""
+    elements, by = sum(numels), {}
+    for e, k in zip(usable, numels):
+        if e is not None:
+            by[e[6]] = by.get(e[6], 0) + k
+    for size, k in by.items():
+        if 2 * k >= elements:
+            return size
+    L = _native.lib()
+    return L.crx_apply_count_slab(elements, L.crx_update_total_changes(u.handle), slab)
+
+
+def _hist_store(t, buf, slab, dev, size):
     """Record counts for t (the caller holds _hist_lock)."""
     key = id(t)
     e = _hist.get(key)
     ref = e[0] if e is not None and e[0]() is t else weakref.ref(t, lambda _r, key=key: _hist_forget(key))
-    _hist[key] = (ref, t._version, buf, slab, dev, buf.data_ptr())
+    _hist[key] = (ref, t._version, buf, slab, dev, buf.data_ptr(), size)
 
 
 def _cache_get(checksums, name, t):
@@ -485,25 +502,30 @@ def apply(weights: Mapping[str, torch.Tensor], u: Update, checksums: dict | None
     # exponent counts carried across updates: only for tensors updated in place with a trusted cache
     keep = checksums is not None and staged is targets and _COUNT_CACHE
     slab = int(_SLAB)
-    hist_in, hist_out, bufs = [], [], []
+    hist_in, hist_out, bufs, usable = [], [], [], []
     if keep:
-        # an entry is used for the same tensor object, unmodified since, with the same slab size and
+        # an entry is used for the same tensor object, unmodified since, with the same _SLAB and
         # device, when the tensor's checksum is trusted too (one pass over the tensors)
-        fresh = []
         with _hist_lock:
             hg = _hist.get
-            for i, (a, c, v) in enumerate(zip(targets, has, vers)):
+            for a, c, v in zip(targets, has, vers):
                 e = hg(id(a)) if c else None
-                if e is not None and e[1] == v and e[3] == slab and e[4] == dev and e[0]() is a:
-                    bufs.append(e[2])
-                    hist_in.append(e[5])
-                else:
-                    bufs.append(None)
-                    hist_in.append(0)
-                    fresh.append(i)
+                ok = e is not None and e[1] == v and e[3] == slab and e[4] == dev and e[0]() is a
+                usable.append(e if ok else None)
+    size = _count_slab(u, usable, numels, slab)
+    if keep:
+        fresh = []
+        for i, e in enumerate(usable):
+            if e is not None and e[6] == size:
+                bufs.append(e[2])
+                hist_in.append(e[5])
+            else:
+                bufs.append(None)
+                hist_in.append(0)
+                fresh.append(i)
         hist_out = list(hist_in)
         # tensors without usable counts: one allocation, sliced per tensor
-        fresh = [(i, L.crx_apply_hist_words(targets[i].numel(), slab)) for i in fresh]
+        fresh = [(i, L.crx_apply_hist_words(targets[i].numel(), size)) for i in fresh]
         if fresh:
             block = torch.empty(sum(w for _, w in fresh), dtype=torch.int32, device=dev)
             at, base = 0, block.data_ptr()
@@ -514,11 +536,11 @@ def apply(weights: Mapping[str, torch.Tensor], u: Update, checksums: dict | None
     with torch.cuda.device(dev):
         if ptrs is None or staged is not targets:
             ptrs = array("Q", [a.data_ptr() for a in staged])
-        rc = L.crx_apply_cached(u.handle, payload_dev or None, _native.view_ptr(ptrs),
+        rc = L.crx_apply_counts(u.handle, payload_dev or None, _native.view_ptr(ptrs),
                                 _native.view_u64(array("Q", numels)), _native.view_i32(has), _native.view_u64(vals),
                                 _native.view_ptr(array("Q", hist_in)) if keep else None,
                                 _native.view_ptr(array("Q", hist_out)) if keep else None,
-                                slab, _native.stream_of(dev), ws.fn, None, ctypes.byref(changed), err, 512)
+                                size, slab, _native.stream_of(dev), ws.fn, None, ctypes.byref(changed), err, 512)
     ws.check()
     ws.release()
     if rc != _native.OK:
@@ -543,9 +565,9 @@ def apply(weights: Mapping[str, torch.Tensor], u: Update, checksums: dict | None
             for a, buf, v in zip(targets, bufs, after):
                 e = hg(id(a))
                 if e is not None and e[2] is buf and e[0]() is a:  # the same counts: a new version only
-                    _hist[id(a)] = (e[0], v, buf, slab, dev, e[5])
+                    _hist[id(a)] = (e[0], v, buf, slab, dev, e[5], size)
                 else:
-                    _hist_store(a, buf, slab, dev)
+                    _hist_store(a, buf, slab, dev, size)
     if checksums is not None:  # record the version after our own write
         checksums.update({name: (c, v) for name, c, v in zip(names, header_chk, after)})
     return changed.value

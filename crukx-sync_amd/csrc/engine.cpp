@@ -551,6 +551,22 @@ uint32_t slab_size(int32_t slab) {
     return s / kRow * kRow;
 }
 
+// Elements per slab of a call over `elements` weights with `changes` changes (0: not known yet): the most
+// one wavefront ranks (slab_size), fewer where that would leave the chip idle.  A wavefront streams its
+// slab row after row, so a slab of 65536 takes 160-240 us however few there are; 2000 to 4000 slabs fill
+// the 256 CUs, and more only add per-slab tables (1 KiB each) to scan.  Measured, one encode + apply
+// (ms): 200,000 weights 0.93 in slabs of 65536, 0.58 of 512; 26.6M weights 1.05 / 0.74 of 8192 (0.77 of
+// 4096 and of 16384); 1.5B weights, encode 2.11 / 2.14 of 32768, apply 2.44 / 2.50, so the largest slab
+// is taken from 2^30 weights on.  An update whose larger slabs would average more than 1600 changes
+// takes half the slab: the select pass holds a slab's changes in a 2048-entry LDS list and reads longer
+// ones from HBM (1.5B weights at 3% changed, 1966 per slab: select 2.75 ms, 2.39 in slabs of 32768).
+uint32_t slab_for(int32_t slab_req, uint64_t elements, uint64_t changes) {
+    uint32_t s = 512;
+    while (s < 32768 && elements > (uint64_t)s * 4096) s *= 2;
+    if (elements >= (1ULL << 30) && changes <= elements / 65536 * 1600) s = 65536;
+    return std::min(s, slab_size(slab_req));
+}
+
 // Slab layout and the chunking of the per-tensor histogram scan.
 struct Layout {
     std::vector<TensorDesc> descs;
@@ -1089,7 +1105,9 @@ void encode_parts(const Layout &L, uint64_t limit, uint32_t slab, const int32_t 
 void encode(int32_t n, const uint16_t *const *olds, const uint16_t *const *news, const uint64_t *numels,
             const int32_t *has_cache, const uint64_t *cache_vals, int32_t slab_req, hipStream_t s, Arena &ar,
             crx_encoded &E) {
-    const uint32_t slab = slab_size(slab_req);
+    uint64_t elements = 0;
+    for (int32_t t = 0; t < n; ++t) elements += numels[t];
+    const uint32_t slab = slab_for(slab_req, elements, 0);
     E.n = n;
     E.present.assign(n, 0);
     E.checksum.assign(n, 0);
@@ -1252,7 +1270,6 @@ void encode(int32_t n, const uint16_t *const *olds, const uint16_t *const *news,
 
 // ------------------------------------------------------------------ apply
 // codec.apply (codec.py:578-717) on the device: decode, locate, verify, then write.
-uint32_t apply_slab(int32_t slab_req) { return slab_size(slab_req); }
 
 // The update's device state that its parts share: the decoding tables, the payload, the block table and
 // each block's first payload bit.
@@ -1441,12 +1458,11 @@ void raise_verdict(const Update &u, unsigned int bad, const std::vector<uint64_t
 
 void apply(const Update &u, const uint8_t *payload_dev, uint16_t *const *targets, const uint64_t *numels,
            const int32_t *has_cache, const uint64_t *cache_vals, uint32_t *const *hist_in, uint32_t *const *hist_out,
-           int32_t slab_req, hipStream_t s, Arena &ar, uint64_t *changed) {
+           uint32_t slab, int32_t slab_req, hipStream_t s, Arena &ar, uint64_t *changed) {
     *changed = 0;
     const uint32_t T = (uint32_t)u.tensors.size();
     if (!T) return;
     HostClock hc;
-    const uint32_t slab = apply_slab(slab_req);
     const uint64_t C = u.total_changes;
     Layout L;
     for (uint32_t t = 0; t < T; ++t) {
@@ -1796,30 +1812,40 @@ uint64_t crx_update_total_changes(const crx_update *u) { return u->u.total_chang
 int32_t crx_apply(const crx_update *u, const uint8_t *payload_dev, uint16_t *const *targets, const uint64_t *numels,
                   const int32_t *has_cache, const uint64_t *cache_vals, int32_t slab, void *stream, crx_alloc_fn alloc,
                   void *alloc_ctx, uint64_t *changed, char *err, uint64_t errlen) {
-    *changed = 0;
-    return guarded(err, errlen, [&] {
-        if (!payload_dev && u->u.payload_len && !u->u.payload_host) throw Invalid("payload is not on the host");
-        Arena ar{alloc, alloc_ctx};
-        apply(u->u, payload_dev, targets, numels, has_cache, cache_vals, nullptr, nullptr, slab, (hipStream_t)stream, ar,
-              changed);
-    });
+    uint64_t elements = 0;
+    for (const TensorHeader &t : u->u.tensors) elements += t.numel;
+    return crx_apply_counts(u, payload_dev, targets, numels, has_cache, cache_vals, nullptr, nullptr,
+                            crx_apply_count_slab(elements, u->u.total_changes, slab), slab, stream, alloc, alloc_ctx, changed, err, errlen);
 }
 
 int32_t crx_apply_cached(const crx_update *u, const uint8_t *payload_dev, uint16_t *const *targets,
                          const uint64_t *numels, const int32_t *has_cache, const uint64_t *cache_vals,
                          uint32_t *const *hist_in, uint32_t *const *hist_out, int32_t slab, void *stream,
                          crx_alloc_fn alloc, void *alloc_ctx, uint64_t *changed, char *err, uint64_t errlen) {
+    return crx_apply_counts(u, payload_dev, targets, numels, has_cache, cache_vals, hist_in, hist_out,
+                            (int32_t)slab_size(slab), slab, stream, alloc, alloc_ctx, changed, err, errlen);
+}
+
+int32_t crx_apply_counts(const crx_update *u, const uint8_t *payload_dev, uint16_t *const *targets,
+                         const uint64_t *numels, const int32_t *has_cache, const uint64_t *cache_vals,
+                         uint32_t *const *hist_in, uint32_t *const *hist_out, int32_t count_slab, int32_t slab,
+                         void *stream, crx_alloc_fn alloc, void *alloc_ctx, uint64_t *changed, char *err,
+                         uint64_t errlen) {
     *changed = 0;
     return guarded(err, errlen, [&] {
         if (!payload_dev && u->u.payload_len && !u->u.payload_host) throw Invalid("payload is not on the host");
         Arena ar{alloc, alloc_ctx};
-        apply(u->u, payload_dev, targets, numels, has_cache, cache_vals, hist_in, hist_out, slab, (hipStream_t)stream,
-              ar, changed);
+        apply(u->u, payload_dev, targets, numels, has_cache, cache_vals, hist_in, hist_out, slab_size(count_slab), slab,
+              (hipStream_t)stream, ar, changed);
     });
 }
 
+int32_t crx_apply_count_slab(uint64_t elements, uint64_t changes, int32_t slab) {
+    return (int32_t)slab_for(slab, elements, changes);
+}
+
 uint64_t crx_apply_hist_words(uint64_t numel, int32_t slab) {
-    const uint32_t sl = apply_slab(slab);
+    const uint32_t sl = slab_size(slab);
     return (numel + sl - 1) / sl * 256;
 }
 

@@ -30,7 +30,8 @@
  *   - `slab` is the reference's codec._SLAB (codec.py:30; 0 = its default, 2^24).  As there, apply
  *     checks the group sizes of tensors of more than `slab` elements before decoding (codec.py:598-604,
  *     "group has more changes than elements").  It also bounds the elements ranked by one wavefront:
- *     min(slab, 65536) rounded down to a multiple of 128 (at least 128).  It never changes the bytes.
+ *     min(slab, 65536) rounded down to a multiple of 128 (at least 128); small calls take fewer
+ *     (crx_apply_count_slab).  It never changes the bytes.
  */
 #ifndef CRUKX_H
 #define CRUKX_H
@@ -136,7 +137,20 @@ int32_t crx_apply_cached(const crx_update *u, const uint8_t *payload_dev, uint16
                          const uint64_t *numels, const int32_t *has_cache, const uint64_t *cache_vals,
                          uint32_t *const *hist_in, uint32_t *const *hist_out, int32_t slab, void *stream,
                          crx_alloc_fn alloc, void *alloc_ctx, uint64_t *changed, char *err, uint64_t errlen);
-/* Size in u32 of one tensor's counts for crx_apply_cached. */
+/* crx_apply_cached with the elements ranked by one wavefront (the slab size of the counts) given by
+ * itself: `count_slab`, a multiple of 128 of at most 65536, instead of the most that `slab` allows
+ * (`slab` then only says which tensors get the group-size check).  hist_in and hist_out hold
+ * crx_apply_hist_words(numel, count_slab) u32. */
+int32_t crx_apply_counts(const crx_update *u, const uint8_t *payload_dev, uint16_t *const *targets,
+                         const uint64_t *numels, const int32_t *has_cache, const uint64_t *cache_vals,
+                         uint32_t *const *hist_in, uint32_t *const *hist_out, int32_t count_slab, int32_t slab,
+                         void *stream, crx_alloc_fn alloc, void *alloc_ctx, uint64_t *changed, char *err,
+                         uint64_t errlen);
+/* The count_slab that suits an update of `changes` changes of tensors of `elements` elements together:
+ * the most that `slab` allows for large ones, fewer where that would leave the chip idle or a slab with
+ * more changes than the select pass keeps on the chip (crx_apply uses it). */
+int32_t crx_apply_count_slab(uint64_t elements, uint64_t changes, int32_t slab);
+/* Size in u32 of one tensor's counts for crx_apply_cached (crx_apply_counts: with its count_slab). */
 uint64_t crx_apply_hist_words(uint64_t numel, int32_t slab);
 
 /* ------------------------------------------------------------------ encode (device)

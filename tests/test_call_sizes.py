@@ -1,0 +1,66 @@
+"""Calls of different sizes take different slab sizes (crx_apply_count_slab) and kernels: results are the
+oracle's at the sizes where the choice changes."""
+
+import pytest
+import torch
+
+import crukx_sync
+import oracle
+import scenarios
+from crukx_sync import _native, codec
+
+
+def _cuda(d):
+    return {k: v.to("cuda") for k, v in d.items()}
+
+
+def test_count_slab_follows_the_size():
+    """Slabs grow with the call, are multiples of a 128-element row, stay within _SLAB, and are halved
+    for updates whose largest slabs would average more than 1600 changes."""
+    def f(elements, slab, changes=0):
+        return _native.lib().crx_apply_count_slab(elements, changes, slab)
+
+    sizes = [f(1 << k, 1 << 24) for k in range(33)]
+    assert sizes == sorted(sizes) and sizes[0] == 512 and sizes[-1] == 65536
+    assert all(s % 128 == 0 for s in sizes)
+    assert f(512 * 4096, 1 << 24) == 512 and f(512 * 4096 + 1, 1 << 24) == 1024
+    assert f(1 << 32, 1 << 24, 65536 * 1600) == 65536 and f(1 << 32, 1 << 24, 65536 * 1600 + 1) == 32768
+    assert [f(1 << 32, s) for s in (1, 128, 1000, 4096, 1 << 14)] == [128, 128, 896, 4096, 1 << 14]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 511, 512, 513, 70_001, 512 * 4096, 512 * 4096 + 1])
+def test_bytes_and_apply_at_slab_edges(n):
+    a, b = scenarios.rl_pair(n, lr=4e-6, seed=n)
+    b[-1] = (b[-1:].view(torch.int16) + 1).view(torch.bfloat16)[0]  # at least one change, in the last slab
+    old, new = {"w": a}, {"w": b}
+    upd = crukx_sync.encode_update(_cuda(old), _cuda(new))
+    assert upd == oracle.encode_update(old, new)
+    recv = _cuda(old)
+    crukx_sync.apply_update(recv, upd)
+    assert torch.equal(recv["w"].cpu().view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.gpu
+def test_counts_kept_while_updates_hold_more_and_fewer_tensors():
+    """Updates of all of a receiver's tensors and of its smallest alone, in turn: each is exact, and the
+    counts of the many stay in use for the few (one slab size), while a receiver that knows only the few
+    takes the many's slab size for all."""
+    shapes = {"big": 3_000_001, "small": 20_003}
+    states = [{}, {}]
+    for i, (k, n) in enumerate(shapes.items()):
+        states[0][k], states[1][k] = scenarios.rl_pair(n, lr=4e-6, seed=900 + i)
+    for first in ("small", "all"):
+        cur = dict(states[0])
+        recv, chk = _cuda(cur), {}
+        sizes = []
+        for which in (first, "all", "small", "all"):
+            nxt = {k: (states[1][k] if cur[k] is states[0][k] else states[0][k]) if which in ("all", k) else cur[k]
+                   for k in shapes}
+            crukx_sync.apply_update(recv, crukx_sync.encode_update(_cuda(cur), _cuda(nxt)), chk)
+            for k in shapes:
+                assert torch.equal(recv[k].cpu().view(torch.int16), nxt[k].view(torch.int16)), (first, which, k)
+            sizes.append(codec._hist[id(recv["small"])][6])
+            cur = nxt
+        assert sizes == ([512, 1024, 1024, 1024] if first == "small" else [1024] * 4)
+        assert {k: v[0] for k, v in chk.items()} == {k: codec.checksum(recv[k]) for k in shapes}
