@@ -1275,6 +1275,7 @@ void encode(int32_t n, const uint16_t *const *olds, const uint16_t *const *news,
 // each block's first payload bit.
 struct ApplyShared {
     uint32_t *lim = nullptr, *off = nullptr, *syms = nullptr;
+    const uint8_t *lens = nullptr;
     uint32_t n_syms = 0, n_tables = 0;
     const uint64_t *pay = nullptr;  // the words holding the payload, from bit bit0 of the first
     uint64_t pay_words = 0;
@@ -1347,7 +1348,7 @@ PartCheck apply_part(const Update &u, const Layout &L, const ApplyPart &P, const
     hc.mark("apply_upload");
     Fork fork(s);
     DecodeArgs da{d_descs, sh.pay, sh.pay_words, sh.bb + P.b0, sh.boff + P.b0, B, d_groups, (uint32_t)G, bmap,
-                  sh.lim, sh.off, sh.syms, sh.n_syms, dz, blk_sum, bad, sh.n_tables, sh.bit0};
+                  sh.lim, sh.off, sh.syms, sh.n_syms, dz, blk_sum, bad, sh.n_tables, sh.bit0, sh.lens};
     launch_decode(da, fork.aux);
     launch_scan_u64(blk_sum, B, blk_prefix, ar.get<unsigned long long>(scan_parts(B)), fork.aux);
 
@@ -1543,12 +1544,25 @@ void apply(const Update &u, const uint8_t *payload_dev, uint16_t *const *targets
 
     ApplyShared sh;
     UploadBatch tb;  // the decoding tables, in one copy
+    // code lengths by a code's first bits, for the decoder that small updates (or parts) take
+    std::vector<uint8_t> lens;
+    for (const ApplyPart &P : parts)
+        if (P.B <= kDecWaveBlocks && lens.empty()) lens.assign(u.tables.size() * kPeekLens, 0);
+    for (size_t ti = 0; ti < lens.size() / kPeekLens; ++ti) {
+        uint32_t from = 0;  // the codes of up to kPeekBits bits end at multiples of one peek
+        for (uint32_t l = 1; l <= kPeekBits; ++l) {
+            const uint32_t to = lim[ti * 17 + l - 1] >> (kMaxCodeLen - kPeekBits);
+            std::fill(lens.begin() + ti * kPeekLens + from, lens.begin() + ti * kPeekLens + to, (uint8_t)l);
+            from = to;
+        }
+    }
     const size_t i_lim = tb.add(lim.data(), lim.size()), i_off = tb.add(off.data(), off.size()),
-                 i_syms = tb.add(syms.data(), syms.size());
+                 i_syms = tb.add(syms.data(), syms.size()), i_lens = tb.add(lens.data(), lens.size());
     tb.commit(ar, s);
     sh.lim = tb.at<uint32_t>(i_lim);
     sh.off = tb.at<uint32_t>(i_off);
     sh.syms = tb.at<uint32_t>(i_syms);
+    sh.lens = tb.at<uint8_t>(i_lens);
     sh.n_syms = (uint32_t)syms.size();
     sh.n_tables = (uint32_t)(lim.size() / 17);
     sh.bb = ar.get<uint32_t>(B_all);

@@ -122,6 +122,8 @@ struct CodeArgs {
     uint64_t bit_base;              // payload bit of these changes' first bit (a part of a chunked update)
 };
 
+constexpr uint32_t kPeekBits = 10, kPeekLens = 1u << kPeekBits;
+
 struct DecodeArgs {
     const TensorDesc *descs;
     // the payload: a big-endian byte stream that starts bit0 bits into the 8-byte aligned word
@@ -143,6 +145,9 @@ struct DecodeArgs {
     unsigned int *bad;
     uint32_t n_tables;              // tables: lim and off hold 17 entries each
     uint32_t bit0;                  // first payload bit in payload[0] (0-56, a multiple of 8)
+    // [tables][kPeekLens], for updates of at most kDecWaveBlocks blocks: the length of the code whose first
+    // kPeekBits bits are the index, or 0 when it is longer (or there is none)
+    const uint8_t *lens;
 };
 
 struct SelectArgs {
@@ -248,6 +253,7 @@ void launch_verdict(uint32_t n, const unsigned long long *delta, const uint64_t 
 void launch_tensor_sums(const TensorDesc *descs, uint32_t n_tensors, const uint64_t *per_tile, uint64_t *out,
                         hipStream_t s);
 void launch_decode(const DecodeArgs &a, hipStream_t s);
+constexpr uint64_t kDecWaveBlocks = 12288;  // updates of up to so many blocks: a wavefront per block
 constexpr uint32_t kDecSyms = 2048;  // decoding symbols staged in LDS when they fit (with the first indices)
 // Dynamic LDS of the decoder for n_syms symbols.
 inline uint32_t decode_lds_bytes(uint32_t n_syms, uint32_t n_tables) { return n_syms <= kDecSyms ? (n_syms + 17u * n_tables) * 4u : 0u; }

@@ -1303,6 +1303,260 @@ __device__ void decode_blocks(const DecodeArgs &a, const uint32_t *S_syms) {
     if (bad) atomicOr(a.bad, kBadDecode);
 }
 
+// ------------------------------------------------------------------ one wavefront per block
+// A lane decodes its 256 changes one after another, 0.5 us each, so however few blocks an update has, the
+// lane-per-block decoder takes 140 us.  Updates too small to fill the chip with lanes take one
+// wavefront per block instead.  Where a code starts is known only once the codes before it are read, but
+// what a code starting at a given bit would be is not: the lanes compute, for every bit of a segment of
+// the block, where the code after it would begin (kSegBits positions, the payload and the results in
+// LDS).  Composing that map with itself three times gives the position eight codes on, so the starts of
+// every eighth code follow in a chain of 32 LDS reads, the ones between from seven more, one lane per
+// chain.  With every start known, each lane decodes four consecutive changes and a wave scan of their
+// gaps gives the block-relative indices.  Codes that do not fit a 64-bit window (long unary runs) are
+// read from HBM one at a time when a chain reaches them.  It decodes some 2500 bit positions to find 256
+// codes, which only pays while the chip has room.  Measured (400 / 2,000 / 3,900 / 7,800 / 15,600 / 31,000
+// blocks, beside nothing else): 23 / 25 / 44 / 72 / 124 / 233 us, the lane-per-block decoder 142 / 141 / 141 /
+// 142 / 145 / 162; beside the cold histogram pass the two meet at about 12,000 blocks, where the line is.
+constexpr uint32_t kSegBits = 3072;      // bit positions per segment (RL-like blocks take about 2500 bits)
+constexpr uint32_t kSegWords = kSegBits / 32 + 5;
+constexpr uint16_t kLongCode = 0xFFFF;   // next position of a code that does not fit its window (or is none)
+static_assert(kSegBits % 512 == 0 && kSegBits + 64 < kLongCode, "kSegBits");
+
+struct alignas(16) WaveDecodeLds {
+    uint32_t w[kSegWords];      // the segment's payload from the word before its first bit's on, big-endian
+    alignas(16) uint8_t len[kPeekLens];     // code length by the first kPeekBits bits of a code; 0: longer than that
+    uint16_t next[kSegBits];    // position of the code after the one starting here (may pass the segment)
+    uint16_t jump[kSegBits];    // ... after the eight codes starting here; kLongCode: not all in the segment
+    uint32_t code[256];         // each code's position in its segment, then its gap
+    uint32_t zz[256];           // ... its symbol
+    uint32_t off[17];           // the table's first symbol index per code length
+};
+
+static_assert(kPeekLens == 64 * sizeof(uint4), "one load per lane");
+
+// the low 32 bits of (hi:lo) >> (n mod 32)
+__device__ __forceinline__ uint32_t funnel_right(uint32_t hi, uint32_t lo, uint32_t n) {
+    return __builtin_amdgcn_alignbit(hi, lo, n);
+}
+
+// the 64 payload bits from bit pos on (past the stream's last word that word again, as BitReader reads)
+__device__ __forceinline__ uint64_t stream_bits(const DecodeArgs &a, uint64_t pos) {
+    const uint64_t t = pos >> 6, n1 = a.n_words - 1;
+    const uint64_t h = __builtin_bswap64(a.payload[min64(t, n1)]), l = __builtin_bswap64(a.payload[min64(t + 1, n1)]);
+    const uint32_t s = (uint32_t)(pos & 63);
+    return s ? (h << s) | (l >> (64 - s)) : h;
+}
+
+// length of the unary run at pos: exact while it is at most qmax and ends before bit `end`, else larger
+// than qmax or reaching `end`
+__device__ uint64_t unary_run(const DecodeArgs &a, uint64_t pos, uint64_t end, uint64_t qmax) {
+    uint64_t q = 0;
+    for (;;) {
+        const uint64_t y = ~stream_bits(a, pos + q);
+        if (y) return q + (uint64_t)__builtin_clzll(y);
+        q += 64;
+        if (q > qmax || pos + q >= end) return q;
+    }
+}
+
+__global__ __launch_bounds__(64) void k_decode_wave(DecodeArgs a) {
+    __shared__ __attribute__((aligned(16))) WaveDecodeLds S;
+    const uint32_t ln = lane();
+    const uint64_t b = blockIdx.x;
+    const GroupDev gr = a.groups[a.bmap[b]];
+    const uint64_t kb = b - gr.blk_base;
+    const uint32_t cnt = (uint32_t)min64(256, gr.count - kb * 256);
+    const uint64_t eb = (uint64_t)gr.elem_base + kb * 256;
+    const uint64_t size = a.descs[gr.tensor].numel;
+    const uint32_t rice = gr.rice;
+    const uint64_t qmax = size >> rice;
+    const uint64_t first = a.bit0 + a.block_off[b], nbits = a.block_bits[b], end = first + nbits;
+    const uint32_t *const lims = a.lim + (uint64_t)gr.table * 17;
+    uint32_t lim[17];  // uniform
+#pragma unroll
+    for (int l = 0; l < 17; ++l) lim[l] = lims[l];
+    if (ln < 17) S.off[ln] = a.off[(uint64_t)gr.table * 17 + ln];
+    reinterpret_cast<uint4 *>(S.len)[ln] = reinterpret_cast<const uint4 *>(a.lens + (uint64_t)gr.table * kPeekLens)[ln];
+    auto length_of = [&](uint32_t peek) -> uint32_t {  // 1 + #{l : lim[l] <= peek}; 18: no code
+        uint32_t L = 1;
+#pragma unroll
+        for (int l = 0; l < 17; ++l) L += lim[l] <= peek ? 1u : 0u;
+        return L;
+    };
+    // remainder and Huffman code at x (the bits after a unary run of q): the change's gap and symbol, and
+    // the length of the two
+    auto finish = [&](uint64_t q, uint64_t x, uint64_t &gap, uint32_t &zz) -> uint32_t {
+        gap = (q << rice) | (rice ? x >> (64 - rice) : 0ULL);
+        const uint32_t peek = (uint32_t)((x << rice) >> (64 - 17)), L = length_of(peek), li = min(L - 1, 16u);
+        const uint32_t idx = S.off[li] + (peek >> (16 - li));
+        zz = a.syms[min(idx, a.n_syms - 1)];
+        return rice + L;
+    };
+    uint32_t done = 0;  // codes decoded
+    uint64_t rel = 0;   // bits of the block before the next code
+    bool bad = false;   // uniform
+    bool off = false;   // this lane decoded a gap past the tensor
+    while (done < cnt && !bad) {  // a segment: at least one code each
+        if (rel >= nbits) {
+            bad = true;
+            break;
+        }
+        // positions [0, n) of the segment are decoded (whole rounds of 512), from bit `at` of the stream
+        const uint64_t at = first + rel, w0 = at >> 5;
+        const uint32_t shift = (uint32_t)(at & 31), n = (uint32_t)min64(kSegBits, (nbits - rel + 511) & ~511ULL);
+        const uint32_t *const p32 = reinterpret_cast<const uint32_t *>(a.payload);
+        const uint64_t n32 = 2 * a.n_words;
+        for (uint32_t i = ln; i < n / 32 + 4; i += 64) S.w[i + 1] = __builtin_bswap32(p32[min64(w0 + i, n32 - 1)]);
+        wave_fence();
+        // position 64 i + ln starts at the same bit s of its word for every i.  Its 64-bit window is two
+        // 32-bit funnel shifts by 32 - s, of the words from the one before it on where s is 0; a unary run
+        // that fills the first 32 bits is left to the chains.
+        const uint32_t s = (shift + ln) & 31, wl = (shift + ln + 31) >> 5, rs = 32 - s;
+        for (uint32_t i0 = 0; i0 < n / 64; i0 += 4) {
+            uint32_t len[4], peek[4], fixed[4];
+            bool any = false;
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                const uint32_t *const w = &S.w[wl + 2 * (i0 + u)];
+                const uint32_t hi = funnel_right(w[0], w[1], rs), lo = funnel_right(w[1], w[2], rs);
+                const uint32_t q = ~hi ? (uint32_t)__builtin_clz(~hi) : 32u;
+                fixed[u] = q + 1 + rice;
+                peek[u] = (uint32_t)(((((uint64_t)hi << 32) | lo) << min(fixed[u], 63u)) >> 47);
+                len[u] = S.len[peek[u] >> (17 - kPeekBits)];
+                if (q == 32 || fixed[u] > 47) len[u] = 18;
+                any = any || len[u] == 0;
+            }
+            if (ballot(any)) {
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u) len[u] = len[u] ? len[u] : length_of(peek[u]);
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                const uint32_t p = 64 * (i0 + u) + ln;
+                S.next[p] = (uint16_t)(len[u] <= 17 ? p + fixed[u] + len[u] : (uint32_t)kLongCode);
+            }
+        }
+        wave_fence();
+        // jump = next composed with itself three times.  A code begins after the one before it, so an
+        // in-place round in ascending order reads only entries that it has not written yet.
+        for (int round = 0; round < 3; ++round) {
+            const uint16_t *const src = round ? S.jump : S.next;
+            for (uint32_t i0 = 0; i0 < n / 64; i0 += 8) {
+                uint32_t m[8], v[8];
+#pragma unroll
+                for (uint32_t u = 0; u < 8; ++u) m[u] = src[64 * (i0 + u) + ln];
+#pragma unroll
+                for (uint32_t u = 0; u < 8; ++u) v[u] = m[u] < n ? src[m[u]] : (uint32_t)kLongCode;
+                wave_fence();
+#pragma unroll
+                for (uint32_t u = 0; u < 8; ++u) S.jump[64 * (i0 + u) + ln] = (uint16_t)v[u];
+                wave_fence();
+            }
+        }
+        // the starts of every eighth code: lane c keeps chain c's
+        uint32_t pos = 0, chains = 0, mine = 0;
+        while (done + 8 * chains + 8 <= cnt && pos < n) {
+            const uint32_t to = __builtin_amdgcn_readfirstlane(S.jump[pos]);
+            if (to == kLongCode) break;
+            if (ln == chains) mine = pos;
+            pos = to;
+            ++chains;
+        }
+        if (ln < chains) {
+            uint32_t c = mine;
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u) {
+                S.code[done + 8 * ln + u] = c;
+                c = S.next[c];
+            }
+        }
+        // then one at a time: the last codes of the block or segment, and a long one
+        uint32_t found = done + 8 * chains;
+        bool is_long = false;
+        while (found < cnt && pos < n) {
+            const uint32_t to = __builtin_amdgcn_readfirstlane(S.next[pos]);
+            is_long = to == kLongCode;
+            if (is_long) break;
+            if (ln == 0) S.code[found] = pos;
+            ++found;
+            pos = to;
+        }
+        wave_fence();
+        // the codes found (the last one again past them), from the payload in LDS; all loads together
+        if (found > done) {
+            uint32_t zz[4];
+            uint64_t gap[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                const uint32_t p = shift + S.code[min(done + 64 * u + ln, found - 1)], *const w = &S.w[(p >> 5) + 1], sh = p & 31;
+                const uint64_t hl = ((uint64_t)w[0] << 32) | w[1], x = sh ? (hl << sh) | (w[2] >> (32 - sh)) : hl;
+                const uint32_t q = (uint32_t)__builtin_clzll(~x);
+                finish(q, x << (q + 1), gap[u], zz[u]);
+                off = off || q > qmax || gap[u] >= size;
+            }
+            wave_fence();
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                const uint32_t i = done + 64 * u + ln;
+                if (i < found) {
+                    S.code[i] = (uint32_t)gap[u];
+                    S.zz[i] = zz[u];
+                }
+            }
+        }
+        done = found;
+        if (is_long) {  // the next segment begins after it
+            const uint64_t cur = at + pos, q = unary_run(a, cur, end, qmax);
+            uint64_t gap = 0;
+            uint32_t zz = 0;
+            bad = q > qmax || cur + q >= end;
+            if (!bad) {
+                const uint32_t len = finish(q, stream_bits(a, cur + q + 1), gap, zz);
+                bad = len > rice + 17 || gap >= size;
+                if (ln == 0) {
+                    S.code[done] = (uint32_t)gap;
+                    S.zz[done] = zz;
+                }
+                ++done;
+                rel += pos + q + 1 + len;
+                pos = 0;
+            }
+        }
+        rel += pos;
+        wave_fence();
+    }
+    // the codes' lengths add up to the block's: each ends inside it
+    const bool far = ballot(off) != 0;
+    bad = bad || rel != nbits || far;
+    unsigned long long sum = 0;
+    if (!bad) {
+        // changes 4 ln .. 4 ln + 3: their gaps summed along the block
+        unsigned long long mine = 0;
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u)
+            if (4 * ln + u < cnt) mine += (unsigned long long)S.code[4 * ln + u] + 1;
+        unsigned long long incl = mine;
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned long long t = __shfl_up(incl, o, 64);
+            if (ln >= (uint32_t)o) incl += t;
+        }
+        sum = __shfl(incl, 63, 64);
+        unsigned long long at = incl - mine;  // sum of (gap + 1) before this lane's changes
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            const uint32_t c = 4 * ln + u;
+            if (c < cnt) {
+                at += (unsigned long long)S.code[c] + 1;
+                a.dz[eb + c] = (unsigned long long)S.zz[c] | ((unsigned long long)min64(at - 1, 0xFFFFFFFFULL) << 32);
+            }
+        }
+    }
+    if (ln == 0) {
+        a.blk_sum[b] = sum;
+        if (bad) atomicOr(a.bad, kBadDecode);
+    }
+}
+
 template <bool LDS_SYMS>
 __global__ __launch_bounds__(64) void k_decode(DecodeArgs a) {
     CRX_DYNAMIC_LDS(uint32_t, dyn_lds);  // the symbols, then the tables' first indices, when they fit
@@ -2250,6 +2504,10 @@ void launch_tensor_sums(const TensorDesc *descs, uint32_t n_tensors, const uint6
 }
 
 void launch_decode(const DecodeArgs &a, hipStream_t s) {
+    if (a.n_blocks <= kDecWaveBlocks) {
+        CRX_LAUNCH("decode", k_decode_wave, (uint32_t)a.n_blocks, 64, s, a);
+        return;
+    }
     const uint32_t grid = grid1(a.n_blocks, 64), lds = decode_lds_bytes(a.n_syms, a.n_tables);
     if (!grid) return;
     timing_begin("decode", s);

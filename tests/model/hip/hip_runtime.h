@@ -202,6 +202,7 @@ inline uint32_t simt_mbcnt_hi(uint32_t m, uint32_t acc) {
 #define __builtin_amdgcn_mbcnt_lo(m, acc) simt_mbcnt_lo((m), (acc))
 #define __builtin_amdgcn_mbcnt_hi(m, acc) simt_mbcnt_hi((m), (acc))
 #define __builtin_amdgcn_readlane(v, l) simt_readlane((v), (l))
+#define __builtin_amdgcn_alignbit(hi, lo, n) ((uint32_t)(((((uint64_t)(hi)) << 32) | (uint32_t)(lo)) >> ((n) & 31u)))
 #define __builtin_amdgcn_readfirstlane(v) simt_readfirstlane((v))
 #define __builtin_amdgcn_fence(order, scope) simt_fence()
 // the emulator's memory operations complete when issued: a wait for them has nothing to wait for

@@ -64,3 +64,50 @@ def test_counts_kept_while_updates_hold_more_and_fewer_tensors():
             cur = nxt
         assert sizes == ([512, 1024, 1024, 1024] if first == "small" else [1024] * 4)
         assert {k: v[0] for k, v in chk.items()} == {k: codec.checksum(recv[k]) for k in shapes}
+
+
+def _many_groups(tensors, n=600):
+    """Every element of `tensors` random int16 tensors changed: 256 groups each, most of one block."""
+    g = torch.Generator().manual_seed(tensors)
+    old = {f"t{i}": torch.randint(-32768, 32768, (n,), generator=g, dtype=torch.int16) for i in range(tensors)}
+    return old, {k: v ^ torch.randint(1, 32768, (n,), generator=g, dtype=torch.int16) for k, v in old.items()}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["host", "device"])
+@pytest.mark.parametrize("tensors", [1, 50, 60])
+def test_decoder_by_number_of_blocks(tensors, form):
+    """Updates on both sides of the number of blocks up to which a wavefront decodes a block: exact, and
+    rejected with the weights unchanged when a payload byte is flipped."""
+    old, new = _many_groups(tensors)
+    upd = crukx_sync.encode_update(_cuda(old), _cuda(new))
+    assert upd == oracle.encode_update(old, new)
+    pay = len(upd) - _native.lib().crx_update_payload_len(crukx_sync.parse(upd).handle)
+    recv = _cuda(old)
+    for at in range(pay, len(upd), max(1, (len(upd) - pay) // 40)):
+        bad = bytearray(upd)
+        bad[at] ^= 0x41
+        with pytest.raises(crukx_sync.CorruptUpdate):
+            crukx_sync.apply_update(recv, bytes(bad) if form == "host" else
+                                    torch.frombuffer(bad, dtype=torch.uint8).cuda())
+    assert all(torch.equal(recv[k].cpu(), old[k]) for k in old)
+    crukx_sync.apply_update(recv, upd if form == "host" else torch.frombuffer(bytearray(upd), dtype=torch.uint8).cuda())
+    assert all(torch.equal(recv[k].cpu(), new[k]) for k in new)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("spread", [3, 700, 9_001, 120_000])
+def test_blocks_of_long_codes(spread):
+    """Blocks of one to many decoder segments, with unary runs past a 64-bit window: changes in dense runs
+    and `spread` elements apart in one exponent group, whose Rice parameter suits neither."""
+    n = 256 * spread + 2048
+    a = torch.full((n,), 0x3F80, dtype=torch.int16)
+    b = a.clone()
+    b[:2048] += 1
+    b[2048::spread] += 3
+    old, new = {"w": a}, {"w": b}
+    upd = crukx_sync.encode_update(_cuda(old), _cuda(new))
+    assert upd == oracle.encode_update(old, new)
+    recv = _cuda(old)
+    crukx_sync.apply_update(recv, upd)
+    assert torch.equal(recv["w"].cpu(), b)
