@@ -148,17 +148,24 @@ hipStream_t aux_stream(hipStream_t caller) {
     return st;
 }
 
+// Without `apart` it is the caller's stream itself, in order.
 struct Fork {
     hipStream_t main, aux;
     hipEvent_t ev[2] = {nullptr, nullptr};
     bool joined = false;
-    explicit Fork(hipStream_t s) : main(s), aux(aux_stream(s)) {
+    Fork(hipStream_t s, bool apart) : main(s), aux(s) {
+        if (!apart) {
+            joined = true;
+            return;
+        }
+        aux = aux_stream(s);
         HIP_OK(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
         HIP_OK(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming));
         HIP_OK(hipEventRecord(ev[0], main));
         HIP_OK(hipStreamWaitEvent(aux, ev[0], 0));
     }
     void join() {
+        if (joined) return;
         HIP_OK(hipEventRecord(ev[1], aux));
         HIP_OK(hipStreamWaitEvent(main, ev[1], 0));
         joined = true;
@@ -167,8 +174,8 @@ struct Fork {
         // an exception before join(): the caller's stream still waits for the auxiliary work, which
         // uses buffers the caller frees after the call
         if (!joined && hipEventRecord(ev[1], aux) == hipSuccess) (void)hipStreamWaitEvent(main, ev[1], 0);
-        (void)hipEventDestroy(ev[0]);
-        (void)hipEventDestroy(ev[1]);
+        for (hipEvent_t e : ev)
+            if (e) (void)hipEventDestroy(e);
     }
 };
 
@@ -510,7 +517,7 @@ void sync(hipStream_t s) {
 struct UploadBatch {
     struct Item {
         const void *src;  // nullptr: zeros
-        uint64_t off, bytes;
+        uint64_t off, bytes, padded;  // zeros follow up to `padded` bytes
     };
     std::vector<Item> items;
     uint64_t total = 0;
@@ -518,8 +525,15 @@ struct UploadBatch {
 
     template <typename T>
     size_t add(const T *src, uint64_t n) {
-        items.push_back({src, total, n * sizeof(T)});
+        items.push_back({src, total, n * sizeof(T), n * sizeof(T)});
         total += (std::max<uint64_t>(n * sizeof(T), 1) + 255) & ~uint64_t(255);
+        return items.size() - 1;
+    }
+    // n elements of src, then zeros to `padded` bytes
+    template <typename T>
+    size_t add_padded(const T *src, uint64_t n, uint64_t padded) {
+        items.push_back({src, total, n * sizeof(T), padded});
+        total += (std::max<uint64_t>(padded, 1) + 255) & ~uint64_t(255);
         return items.size() - 1;
     }
     template <typename T>
@@ -529,7 +543,7 @@ struct UploadBatch {
         uint8_t *p = t_stage.get(total);
         for (const Item &it : items) {
             if (it.src) std::memcpy(p + it.off, it.src, it.bytes);
-            else std::memset(p + it.off, 0, it.bytes);
+            std::memset(p + it.off + (it.src ? it.bytes : 0), 0, it.padded - (it.src ? it.bytes : 0));
         }
         HIP_OK(hipMemcpyAsync(dev, p, total, hipMemcpyHostToDevice, s));
         t_stage.copied(s);
@@ -572,14 +586,22 @@ struct Layout {
     std::vector<TensorDesc> descs;
     std::vector<int32_t> call_index;  // descriptor -> caller's tensor index
     uint32_t tiles = 0;
-    std::vector<ScanChunk> chunks;
-    std::vector<uint32_t> tensor_chunk_begin;
+    std::vector<ScanCols> cols;         // the scan's plan: columns of every tensor, or (a tensor of more than
+    std::vector<ScanChunk> chunks;      // kScanTensorTiles slabs) chunks of every tensor and the tensors'
+    std::vector<uint32_t> tensor_chunk_begin;  // first chunks
+    std::vector<uint32_t> tile_tensor;  // the slabs' tensors, of few enough slabs to upload them
 };
+// Up to so many slabs the slab-to-tensor map is built on the host and goes with the call's other small
+// uploads (64 KiB at most) instead of in a launch of its own.
+constexpr uint32_t kHostTileMap = 16384;
 
 void finish_layout(Layout &L, uint32_t slab) {
     L.tiles = 0;
+    L.cols.clear();
     L.chunks.clear();
     L.tensor_chunk_begin.assign(1, 0);
+    L.tile_tensor.clear();
+    uint32_t most = 0;  // slabs of the tensor with the most
     for (uint32_t t = 0; t < L.descs.size(); ++t) {
         TensorDesc &d = L.descs[t];
         uint64_t nt = (d.numel + slab - 1) / slab;
@@ -587,11 +609,22 @@ void finish_layout(Layout &L, uint32_t slab) {
         d.tile_begin = L.tiles;
         d.n_tiles = (uint32_t)nt;
         L.tiles += (uint32_t)nt;
-        for (uint32_t c = 0; c < nt; c += kScanTiles)
-            L.chunks.push_back(
-                ScanChunk{d.tile_begin + c, d.tile_begin + std::min<uint32_t>(c + kScanTiles, (uint32_t)nt), t, 0});
-        L.tensor_chunk_begin.push_back((uint32_t)L.chunks.size());
+        most = std::max(most, (uint32_t)nt);
     }
+    for (uint32_t t = 0; t < L.descs.size(); ++t) {
+        const TensorDesc &d = L.descs[t];
+        if (most <= kScanTensorTiles) {
+            const uint32_t n = d.n_tiles <= kScanFewTiles ? 256 : kScanFewCols;
+            for (uint32_t k = 0; k < 256; k += n) L.cols.push_back(ScanCols{t, k, n, 0});
+        } else {
+            for (uint32_t c = 0; c < d.n_tiles; c += kScanTiles)
+                L.chunks.push_back(ScanChunk{d.tile_begin + c,
+                                             d.tile_begin + std::min<uint32_t>(c + kScanTiles, d.n_tiles), t, 0});
+            L.tensor_chunk_begin.push_back((uint32_t)L.chunks.size());
+        }
+    }
+    if (L.tiles <= kHostTileMap)
+        for (uint32_t t = 0; t < L.descs.size(); ++t) L.tile_tensor.insert(L.tile_tensor.end(), L.descs[t].n_tiles, t);
 }
 
 TensorDesc make_desc(const uint16_t *p, uint64_t numel) {
@@ -605,27 +638,40 @@ TensorDesc make_desc(const uint16_t *p, uint64_t numel) {
     return d;
 }
 
-// Device copies of the scan chunking.
+// Device copies of a layout's scan plan and slab-to-tensor map.
 struct ScanDev {
-    ScanChunk *chunks;
-    uint32_t *tcb, *csum;
-    uint32_t n_chunks;
+    ScanPlan plan;
+    uint32_t *csum;         // [chunks][256]
     uint32_t *tile_tensor;  // [tiles]
 };
 
-// The scan's tables on the device, with its chunk list and the tensors' first chunks already uploaded
-// (chunks, tcb); the slab-to-tensor map is built here.
-ScanDev scan_buffers(Arena &ar, const Layout &L, const TensorDesc *d_descs, ScanChunk *chunks, uint32_t *tcb,
-                     hipStream_t s) {
-    ScanDev sd;
-    sd.tile_tensor = ar.get<uint32_t>(L.tiles);
-    launch_tile_map(d_descs, (uint32_t)L.descs.size(), sd.tile_tensor, s);
-    sd.n_chunks = (uint32_t)L.chunks.size();
-    sd.chunks = chunks;
-    sd.tcb = tcb;
-    sd.csum = ar.get<uint32_t>((uint64_t)sd.n_chunks * 256);
-    return sd;
-}
+// The layout's arrays that go to the device with the call's other small uploads.
+struct LayoutUpload {
+    size_t cols, chunks, tcb, tiles;
+    LayoutUpload(UploadBatch &ub, const Layout &L)
+        : cols(ub.add(L.cols.data(), L.cols.size())), chunks(ub.add(L.chunks.data(), L.chunks.size())),
+          tcb(ub.add(L.tensor_chunk_begin.data(), L.tensor_chunk_begin.size())),
+          tiles(ub.add(L.tile_tensor.data(), L.tile_tensor.size())) {}
+    // once they are uploaded (a slab-to-tensor map too large for that is built here)
+    ScanDev on_device(const UploadBatch &ub, Arena &ar, const Layout &L, const TensorDesc *d_descs, hipStream_t s) const {
+        ScanDev sd;
+        sd.tile_tensor = ub.at<uint32_t>(tiles);
+        if (L.tile_tensor.empty()) {
+            sd.tile_tensor = ar.get<uint32_t>(L.tiles);
+            launch_tile_map(d_descs, (uint32_t)L.descs.size(), sd.tile_tensor, s);
+        }
+        if (!L.cols.empty()) {
+            sd.plan.cols = ub.at<ScanCols>(cols);
+            sd.plan.n_cols = (uint32_t)L.cols.size();
+        } else {
+            sd.plan.chunks = ub.at<ScanChunk>(chunks);
+            sd.plan.tcb = ub.at<uint32_t>(tcb);
+            sd.plan.n_chunks = (uint32_t)L.chunks.size();
+        }
+        sd.csum = ar.get<uint32_t>((uint64_t)L.chunks.size() * 256);
+        return sd;
+    }
+};
 
 }  // namespace crx
 
@@ -816,22 +862,20 @@ struct Ranked {
 Ranked rank_changes(const Layout &L, uint32_t slab, hipStream_t s, Arena &ar, HostClock *hc, uint64_t stop_at) {
     const uint32_t T = (uint32_t)L.descs.size(), tiles = L.tiles;
     Ranked R;
-    UploadBatch ub;  // the tensors, the scan's chunks and a zeroed overflow flag in one copy
-    const size_t i_descs = ub.add(L.descs.data(), T), i_chunks = ub.add(L.chunks.data(), L.chunks.size()),
-                 i_tcb = ub.add(L.tensor_chunk_begin.data(), L.tensor_chunk_begin.size()),
-                 i_ovf = ub.add_zeros<unsigned int>(1);
+    UploadBatch ub;  // the tensors, the scan's plan and a zeroed overflow flag in one copy
+    const size_t i_descs = ub.add(L.descs.data(), T), i_ovf = ub.add_zeros<unsigned int>(1);
+    const LayoutUpload lu(ub, L);
     ub.commit(ar, s);
     R.d_descs = ub.at<TensorDesc>(i_descs);
     R.hall = ar.get<uint32_t>((uint64_t)tiles * 256);
     R.hchg = ar.get<uint32_t>((uint64_t)tiles * 256);
     R.delta = ar.get<uint64_t>(tiles);
     R.full = ar.get<uint64_t>(tiles);
-    R.sd = scan_buffers(ar, L, R.d_descs, ub.at<ScanChunk>(i_chunks), ub.at<uint32_t>(i_tcb), s);
+    R.sd = lu.on_device(ub, ar, L, R.d_descs, s);
     uint32_t *tot_all = ar.get<uint32_t>((uint64_t)T * 256), *tot_chg = ar.get<uint32_t>((uint64_t)T * 256);
-    uint32_t *csum_chg = ar.get<uint32_t>((uint64_t)R.sd.n_chunks * 256);  // the change counts' chunk sums
+    uint32_t *csum_chg = ar.get<uint32_t>((uint64_t)R.sd.plan.n_chunks * 256);  // the change counts' chunk sums
     R.d_groups = ar.get<GroupDev>((uint64_t)T * 256);
     R.gbase = ar.get<uint32_t>((uint64_t)T * 256);
-    unsigned long long *gcnt = ar.get<unsigned long long>(2);
 
     // Each slab stores its change records in a region of its own, sized for 1/24 of its elements
     // (+64).  If one overflows, the exact counts of that pass give exact regions for a second pass.
@@ -845,18 +889,17 @@ Ranked rank_changes(const Layout &L, uint32_t slab, hipStream_t s, Arena &ar, Ho
     // the scans and groups need only the counts, which are exact even when a slab's records overflowed
     // their region; the overflow flag is read with the group totals, and on overflow the rank pass runs
     // again into exact regions (rewriting the counts, so they are scanned again)
-    unsigned int hovf1 = 0;
-    unsigned long long gc[2];
     for (int pass = 0;; ++pass) {
         const ScanTabs tabs{{R.hall, R.hchg}, {R.sd.csum, csum_chg}, {tot_all, tot_chg}};
-        launch_scan_tables(R.d_descs, tabs, 2, R.sd.chunks, R.sd.n_chunks, R.sd.tcb, T, s);
-        launch_enc_groups(tot_chg, T, R.d_groups, R.gbase, gcnt, s);
-        d2h(&hovf1, ovf, 1, s);
-        d2h(gc, gcnt, 2, s);
+        launch_scan_tables(R.d_descs, tabs, 2, R.sd.plan, T, s);
+        // groups, changes and the overflow flag, written by the kernel into pinned memory (no copy)
+        auto *result = reinterpret_cast<volatile unsigned long long *>(t_stage.get(3 * sizeof(unsigned long long)));
+        launch_enc_groups(tot_chg, T, R.d_groups, R.gbase, ovf, const_cast<unsigned long long *>(result), s);
+        t_stage.copied(s);
         sync(s);
-        R.G = gc[0];
-        R.C = gc[1];
-        if (!hovf1 || R.C >= stop_at) break;
+        R.G = result[0];
+        R.C = result[1];
+        if (!result[2] || R.C >= stop_at) break;
         if (pass) throw DeviceError("change records overflowed exact regions");
         unsigned long long *rec_base = ar.get<unsigned long long>(tiles + 1);
         launch_scan_u32(rec_count, tiles, rec_base, ar.get<unsigned long long>(scan_parts(tiles)), s);
@@ -966,8 +1009,7 @@ void encode_parts(const Layout &L, uint64_t limit, uint32_t slab, const int32_t 
         const Ranked R = rank_changes(p.L, slab, s, ar, nullptr, UINT64_MAX);
         p.C = R.C;
         uint64_t *t_delta = ar.get<uint64_t>(T), *t_full = ar.get<uint64_t>(T);
-        launch_tensor_sums(R.d_descs, T, R.delta, t_delta, s);
-        launch_tensor_sums(R.d_descs, T, R.full, t_full, s);
+        launch_tensor_sums(R.d_descs, T, R.delta, R.full, t_delta, t_full, s);
         d2h(hdelta.data(), t_delta, T, s);
         d2h(hfull.data(), t_full, T, s);
         unsigned long long hs[2] = {0, 0};
@@ -976,14 +1018,12 @@ void encode_parts(const Layout &L, uint64_t limit, uint32_t slab, const int32_t 
             uint64_t *sorted = ar.get<uint64_t>(R.C);
             launch_place(R.a, p.L.tiles, R.sd.tile_tensor, R.hall, R.hchg, R.gbase, sorted, R.C, s);
             uint32_t *cmap = ar.get<uint32_t>((R.C + kElemsPerThread - 1) / kElemsPerThread);
-            launch_chunk_map(R.d_groups, (uint32_t)R.G, cmap, s);
-            launch_r0(R.d_groups, (uint32_t)R.G, sorted, s);
-            uint32_t *d_dense = ar.get<uint32_t>(256 * kDense);
+            // cost | scnt | dense, cleared together
+            unsigned long long *cost = ar.get<unsigned long long>(R.G * 3 + 2 + 128 * kDense), *scnt = cost + R.G * 3;
+            uint32_t *d_dense = reinterpret_cast<uint32_t *>(scnt + 2);
+            launch_enc_prep(R.d_groups, (uint32_t)R.G, sorted, cmap, nullptr, reinterpret_cast<uint32_t *>(cost),
+                            (uint32_t)(R.G * 6 + 4 + 256 * kDense), s);
             d_rare = ar.get<uint32_t>(R.C);
-            unsigned long long *scnt = ar.get<unsigned long long>(2), *cost = ar.get<unsigned long long>(R.G * 3);
-            zero(d_dense, 256 * kDense, s);
-            zero(scnt, 2, s);
-            zero(cost, R.G * 3, s);
             StatsArgs st{sorted, R.C, R.d_groups, (uint32_t)R.G, cmap, d_dense, d_rare, R.C, scnt, cost};
             launch_stats(st, s);
             p.groups.resize(R.G);
@@ -1074,17 +1114,14 @@ void encode_parts(const Layout &L, uint64_t limit, uint32_t slab, const int32_t 
         h2d(d_groups, p.groups.data(), G, s);
         const uint64_t n_thr = (p.C + kElemsPerThread - 1) / kElemsPerThread;
         uint32_t *cmap = ar.get<uint32_t>(n_thr);
-        launch_chunk_map(d_groups, (uint32_t)G, cmap, s);
+        launch_enc_prep(d_groups, (uint32_t)G, nullptr, cmap, nullptr, nullptr, 0, s);
         unsigned long long *tsum = ar.get<unsigned long long>(n_thr), *toff = ar.get<unsigned long long>(n_thr + 1);
         unsigned long long *bstart = ar.get<unsigned long long>(p.B + 1);
         unsigned int *bovf = ar.get<unsigned int>(1);
         CodeArgs ca{sorted, p.C, d_groups, (uint32_t)G, d_lut, d_rk, d_rv, (uint32_t)rkeys.size(), cmap, tsum, toff,
-                    words, bstart, n_words, bovf, p.bit0};
+                    words, bstart, n_words, bovf, p.bit0, p.B, 0};
         launch_code_lengths(ca, s);
         launch_scan_u64(tsum, n_thr, toff, ar.get<unsigned long long>(scan_parts(n_thr)), s);
-        zero(bovf, 1, s);
-        const unsigned long long end = p.bit0 + p.bits;  // the block starts are payload bits: so is the end
-        h2d(bstart + p.B, &end, 1, s);
         launch_pack(ca, s);
         launch_block_bits(bstart, p.B, bb + p.blk0, bovf, s);
         unsigned int hovf = 0;
@@ -1157,37 +1194,36 @@ void encode(int32_t n, const uint16_t *const *olds, const uint16_t *const *news,
     launch_place(a, tiles, sd.tile_tensor, hall, hchg, gbase, sorted, C, s);
     const uint64_t n_thr = (C + kElemsPerThread - 1) / kElemsPerThread;  // threads of the walking kernels
     uint32_t *cmap = ar.get<uint32_t>(n_thr);
-    launch_chunk_map(d_groups, (uint32_t)G, cmap, s);
-    launch_r0(d_groups, (uint32_t)G, sorted, s);
     // what the host reads back after the symbol counts, in one block so that one copy brings it (the
-    // first kRareFirst rare symbols with it): cost | dense | scnt | t_delta | t_full | rare
-    const uint64_t o_dense = G * 3 * 8, o_scnt = o_dense + 256 * kDense * 4, o_delta = o_scnt + 16,
-                   o_full = o_delta + 8 * (uint64_t)T, o_rare = o_full + 8 * (uint64_t)T;
+    // first kRareFirst rare symbols with it): groups | cost | dense | scnt | t_delta | t_full | rare
+    const uint64_t o_cost = G * sizeof(GroupDev), o_dense = o_cost + G * 3 * 8, o_scnt = o_dense + 256 * kDense * 4,
+                   o_delta = o_scnt + 16, o_full = o_delta + 8 * (uint64_t)T, o_rare = o_full + 8 * (uint64_t)T;
     uint8_t *dl = ar.get<uint8_t>(o_rare + 4 * C);
-    unsigned long long *cost = reinterpret_cast<unsigned long long *>(dl);
+    unsigned long long *cost = reinterpret_cast<unsigned long long *>(dl + o_cost);
     uint32_t *dense = reinterpret_cast<uint32_t *>(dl + o_dense);
     unsigned long long *scnt = reinterpret_cast<unsigned long long *>(dl + o_scnt);
     uint64_t *t_delta = reinterpret_cast<uint64_t *>(dl + o_delta), *t_full = reinterpret_cast<uint64_t *>(dl + o_full);
     uint32_t *rare = reinterpret_cast<uint32_t *>(dl + o_rare);
-    zero(dl, o_delta, s);  // cost, dense and scnt; the sums are written whole
+    // clears cost, dense and scnt; the sums are written whole
+    launch_enc_prep(d_groups, (uint32_t)G, sorted, cmap, reinterpret_cast<GroupDev *>(dl),
+                    reinterpret_cast<uint32_t *>(cost), (uint32_t)((o_delta - o_cost) / 4), s);
     StatsArgs st{sorted, C, d_groups, (uint32_t)G, cmap, dense, rare, C, scnt, cost};
     launch_stats(st, s);
-    launch_tensor_sums(d_descs, T, delta, t_delta, s);
-    launch_tensor_sums(d_descs, T, full, t_full, s);
+    launch_tensor_sums(d_descs, T, delta, full, t_delta, t_full, s);
 
-    std::vector<GroupDev> groups(G);
-    d2h(groups.data(), d_groups, G, s);
     // the first rare symbols in the same wait (an update has few); the rest, if any, after it
     const uint64_t rare_first = std::min<uint64_t>(C, kRareFirst);
     std::vector<uint8_t> hdl(o_rare + 4 * rare_first);
     d2h(hdl.data(), dl, hdl.size(), s);
     sync(s);
     hc.mark("enc_wait_stats");
+    std::vector<GroupDev> groups(G);
     std::vector<unsigned long long> hcost(G * 3);
     std::vector<uint32_t> hdense(256 * kDense);
     std::vector<uint64_t> hdelta(T), hfull(T);
     unsigned long long hs[2];
-    std::memcpy(hcost.data(), hdl.data(), o_dense);
+    std::memcpy(groups.data(), hdl.data(), o_cost);
+    std::memcpy(hcost.data(), hdl.data() + o_cost, o_dense - o_cost);
     std::memcpy(hdense.data(), hdl.data() + o_dense, 256 * kDense * 4);
     std::memcpy(hs, hdl.data() + o_scnt, 16);
     std::memcpy(hdelta.data(), hdl.data() + o_delta, 8 * (uint64_t)T);
@@ -1220,31 +1256,27 @@ void encode(int32_t n, const uint16_t *const *olds, const uint16_t *const *news,
     hc.mark("enc_tables");
 
     // the code lengths, their offsets and the bits, with no wait: the payload's size is known
-    UploadBatch ub;  // the groups with their Rice parameters, the code tables, a zeroed overflow flag
+    UploadBatch ub;  // the groups with their Rice parameters, the code tables
     const size_t i_groups = ub.add(groups.data(), G), i_lut = ub.add(lut.data(), lut.size()),
-                 i_rk = ub.add(rkeys.data(), rkeys.size()), i_rv = ub.add(rvals.data(), rvals.size()),
-                 i_ovf = ub.add_zeros<unsigned int>(1);
+                 i_rk = ub.add(rkeys.data(), rkeys.size()), i_rv = ub.add(rvals.data(), rvals.size());
     ub.commit(ar, s);
     GroupDev *d_groups2 = ub.at<GroupDev>(i_groups);
     uint32_t *d_lut = ub.at<uint32_t>(i_lut), *d_rk = ub.at<uint32_t>(i_rk), *d_rv = ub.at<uint32_t>(i_rv);
-    unsigned long long *tsum = ar.get<unsigned long long>(n_thr), *toff = ar.get<unsigned long long>(n_thr + 1);
+    // the bit offsets, their total, and the flags of the code kernels behind it: one copy brings both back
+    unsigned long long *tsum = ar.get<unsigned long long>(n_thr), *toff = ar.get<unsigned long long>(n_thr + 2);
+    unsigned int *bovf = reinterpret_cast<unsigned int *>(toff + n_thr + 1);
     const uint64_t n_words = (total_bits + 31) / 32 + 4;
     uint32_t *words = ar.get<uint32_t>(n_words);
     unsigned long long *bstart = ar.get<unsigned long long>(B + 1);
     uint32_t *bb = ar.get<uint32_t>(B);
-    unsigned int *bovf = ub.at<unsigned int>(i_ovf);
     CodeArgs ca{sorted, C, d_groups2, (uint32_t)G, d_lut, d_rk, d_rv, (uint32_t)rkeys.size(), cmap, tsum, toff,
-                words, bstart, n_words, bovf};
+                words, bstart, n_words, bovf, 0, B, n_words};
     launch_code_lengths(ca, s);
     launch_scan_u64(tsum, n_thr, toff, ar.get<unsigned long long>(scan_parts(n_thr)), s);
-    zero(words, n_words, s);
-    HIP_OK(hipMemcpyAsync(bstart + B, toff + n_thr, sizeof(unsigned long long), hipMemcpyDeviceToDevice, s));
     launch_pack(ca, s);
     launch_block_bits(bstart, B, bb, bovf, s);
-    unsigned int hovf = 0;
-    unsigned long long dev_bits = 0;
-    d2h(&hovf, bovf, 1, s);
-    d2h(&dev_bits, toff + n_thr, 1, s);
+    unsigned long long last[2] = {0, 0};  // the bits of all codes, the flags
+    d2h(last, toff + n_thr, 2, s);
 
     // the rest of the host's part while the device packs: checksums (codec.py:344-352), the groups
     for (uint32_t d = 0; d < T; ++d) {
@@ -1260,7 +1292,8 @@ void encode(int32_t n, const uint16_t *const *olds, const uint16_t *const *news,
     E.n_blocks = B;
     sync(s);
     hc.mark("enc_wait_pack");
-    if (hovf & 2u || dev_bits != total_bits) throw DeviceError("the packed payload's size differs from its codes' lengths");
+    const unsigned int hovf = (unsigned int)last[1];  // the flags' half of the word
+    if (hovf & 2u || last[0] != total_bits) throw DeviceError("the packed payload's size differs from its codes' lengths");
     if (hovf) throw Invalid("a block exceeds 2^32 bits; the update cannot be represented");
     g_encode_hint.put(hint_key, ar.total);
     E.d_block_bits = bb;
@@ -1270,6 +1303,11 @@ void encode(int32_t n, const uint16_t *const *olds, const uint16_t *const *news,
 
 // ------------------------------------------------------------------ apply
 // codec.apply (codec.py:578-717) on the device: decode, locate, verify, then write.
+
+// A host update's block table and payload of up to so many bytes go with the call's other small uploads
+// (one copy from pinned memory) instead of in copies of their own (7-10 us each, and the host held by
+// those from pageable memory).
+constexpr uint64_t kSmallUpdate = 1ULL << 20;
 
 // The update's device state that its parts share: the decoding tables, the payload, the block table and
 // each block's first payload bit.
@@ -1300,12 +1338,16 @@ struct PartCheck {
     std::vector<uint64_t> delta, full;
 };
 
+constexpr uint32_t kForkTiles = 8192;
+
 // One part of an update, or the whole of it (codec.py:578-717): decode, locate, verify, then write.
 // dry: the part is only verified; nothing is written (no write-through, no commit, and the receiver's
-// exponent counts are not kept up to date).
-PartCheck apply_part(const Update &u, const Layout &L, const ApplyPart &P, const ApplyShared &sh,
-                     const int32_t *has_cache, const uint64_t *cache_vals, uint32_t slab, int32_t slab_req, bool dry,
-                     hipStream_t s, Arena &ar, HostClock &hc) {
+// exponent counts are not kept up to date).  ub: uploads that go with the part's; `uploaded` is called
+// once they are enqueued, and completes `sh`.
+template <typename F>
+PartCheck apply_part(const Update &u, const Layout &L, const ApplyPart &P, const ApplyShared &sh, UploadBatch &ub,
+                     F &&uploaded, const int32_t *has_cache, const uint64_t *cache_vals, uint32_t slab,
+                     int32_t slab_req, bool dry, hipStream_t s, Arena &ar, HostClock &hc) {
     const uint32_t T = (uint32_t)L.descs.size(), tiles = L.tiles;
     const uint64_t G = P.groups.size(), B = P.B, C = P.C;
     std::vector<uint32_t> tensor_chg(T + 1, (uint32_t)C);  // first change of each tensor (its changes are contiguous)
@@ -1326,14 +1368,13 @@ PartCheck apply_part(const Update &u, const Layout &L, const ApplyPart &P, const
     }
 
     // every small upload of the part in one copy, ahead of the decoder, which starts at once
-    UploadBatch ub;
     const size_t i_descs = ub.add(descs.data(), T), i_groups = ub.add(P.groups.data(), G),
                  i_gof = ub.add(P.group_of.data(), P.group_of.size()), i_tchg = ub.add(tensor_chg.data(), T + 1),
-                 i_chunks = ub.add(L.chunks.data(), L.chunks.size()),
-                 i_tcb = ub.add(L.tensor_chunk_begin.data(), L.tensor_chunk_begin.size()),
                  i_want = ub.add(want.data(), T), i_cached = ub.add(cached.data(), T), i_has = ub.add(has.data(), T),
                  i_bad = ub.add_zeros<unsigned int>(1), i_nmore = ub.add_zeros<unsigned int>(1);
+    const LayoutUpload lu(ub, L);
     ub.commit(ar, s);
+    uploaded();
     TensorDesc *d_descs = ub.at<TensorDesc>(i_descs);
     GroupDev *d_groups = ub.at<GroupDev>(i_groups);
     unsigned int *bad = ub.at<unsigned int>(i_bad);
@@ -1342,11 +1383,12 @@ PartCheck apply_part(const Update &u, const Layout &L, const ApplyPart &P, const
     launch_block_map(d_groups, (uint32_t)G, bmap, binfo, s);
 
     // The decoder needs nothing from the receiver's weights: it runs on the auxiliary stream while
-    // the main stream takes the exponent counts (pass A) and their scans.
+    // the main stream takes the exponent counts (pass A) and their scans, where those take longer than the
+    // two streams take to wait for each other (30-40 us: kForkTiles).
     unsigned long long *dz = ar.get<unsigned long long>(C);
     unsigned long long *blk_sum = ar.get<unsigned long long>(B), *blk_prefix = ar.get<unsigned long long>(B + 1);
     hc.mark("apply_upload");
-    Fork fork(s);
+    Fork fork(s, tiles > kForkTiles);
     DecodeArgs da{d_descs, sh.pay, sh.pay_words, sh.bb + P.b0, sh.boff + P.b0, B, d_groups, (uint32_t)G, bmap,
                   sh.lim, sh.off, sh.syms, sh.n_syms, dz, blk_sum, bad, sh.n_tables, sh.bit0, sh.lens};
     launch_decode(da, fork.aux);
@@ -1354,7 +1396,7 @@ PartCheck apply_part(const Update &u, const Layout &L, const ApplyPart &P, const
 
     uint32_t *hall = ar.get<uint32_t>((uint64_t)tiles * 256);
     uint64_t *full = ar.get<uint64_t>(tiles), *t_full = ar.get<uint64_t>(T);
-    ScanDev sd = scan_buffers(ar, L, d_descs, ub.at<ScanChunk>(i_chunks), ub.at<uint32_t>(i_tcb), s);
+    ScanDev sd = lu.on_device(ub, ar, L, d_descs, s);
     uint32_t *sizes = ar.get<uint32_t>((uint64_t)T * 256);
     int32_t *d_gof = ub.at<int32_t>(i_gof);
     uint32_t *local = ar.get<uint32_t>(C);
@@ -1384,7 +1426,7 @@ PartCheck apply_part(const Update &u, const Layout &L, const ApplyPart &P, const
         launch_hist(ha, (uint32_t)hist_list.size(), s);
     }
     const ScanTabs tabs{{hall, nullptr}, {sd.csum, nullptr}, {sizes, nullptr}};
-    launch_scan_tables(d_descs, tabs, 1, sd.chunks, sd.n_chunks, sd.tcb, T, s);
+    launch_scan_tables(d_descs, tabs, 1, sd.plan, T, s);
     fork.join();
     hc.mark("apply_pass_a");
 
@@ -1415,25 +1457,27 @@ PartCheck apply_part(const Update &u, const Layout &L, const ApplyPart &P, const
     launch_select(sa, tiles, C > kSelectDenseTargets * tiles, any_cold, s);
     SlabArgs sla{d_descs, sd.tile_tensor, slab, rstart, rec, dz, pn, sdelta, bad, nullptr, (uint32_t)C, multi, done};
     launch_verify(sla, tiles, s);
-    launch_tensor_sums(d_descs, T, sdelta, tdelta, s);
-    launch_tensor_sums(d_descs, T, full, t_full, s);  // the select pass summed the cold slabs
+    launch_tensor_sums(d_descs, T, sdelta, full, tdelta, t_full, s);  // the select pass summed the cold slabs
+    // the verdict on the device too, and the commit behind it (the remaining writes if the update
+    // verifies, the undoing of the select pass's if not); the host waits for the verdict's data only
+    auto *result = reinterpret_cast<unsigned long long *>(t_stage.get((1 + 2 * (uint64_t)T) * sizeof(unsigned long long)));
+    launch_verdict(T, reinterpret_cast<const unsigned long long *>(tdelta), t_full, d_has, d_cached, d_want, bad, ok,
+                   result, s);
     if (!dry) {
-        // the verdict on the device too, and the commit behind it (the remaining writes if the update
-        // verifies, the undoing of the select pass's if not); the host waits for the verdict's data only
-        launch_verdict(T, reinterpret_cast<const unsigned long long *>(tdelta), t_full, d_has, d_cached, d_want, bad,
-                       ok, s);
         sla.ok = ok;
         launch_commit(sla, tiles, s);  // next to the verdict: nothing on the host can fail in between
     }
+    t_stage.copied(s);
     hc.mark("apply_launch");
 
     PartCheck r;
     r.delta.resize(T);
     r.full.resize(T);
-    d2h(&r.bad, bad, 1, s);
-    d2h(r.delta.data(), tdelta, T, s);
-    d2h(r.full.data(), t_full, T, s);
-    t_stage.finish();  // the downloads above (behind the commit, which exits at once when the update verifies)
+    t_stage.wait();  // behind the commit, which exits at once when the update verifies
+    r.bad = (unsigned int)result[0];
+    std::copy(result + 1, result + 1 + T, r.delta.begin());
+    std::copy(result + 1 + T, result + 1 + 2 * (uint64_t)T, r.full.begin());
+    t_stage.finish();
     hc.mark("apply_wait_verify");
     return r;
 }
@@ -1543,7 +1587,7 @@ void apply(const Update &u, const uint8_t *payload_dev, uint16_t *const *targets
     hc.mark("apply_tables");
 
     ApplyShared sh;
-    UploadBatch tb;  // the decoding tables, in one copy
+    UploadBatch tb;  // the decoding tables, in one copy, and with them a small update's bytes
     // code lengths by a code's first bits, for the decoder that small updates (or parts) take
     std::vector<uint8_t> lens;
     for (const ApplyPart &P : parts)
@@ -1558,58 +1602,70 @@ void apply(const Update &u, const uint8_t *payload_dev, uint16_t *const *targets
     }
     const size_t i_lim = tb.add(lim.data(), lim.size()), i_off = tb.add(off.data(), off.size()),
                  i_syms = tb.add(syms.data(), syms.size()), i_lens = tb.add(lens.data(), lens.size());
-    tb.commit(ar, s);
-    sh.lim = tb.at<uint32_t>(i_lim);
-    sh.off = tb.at<uint32_t>(i_off);
-    sh.syms = tb.at<uint32_t>(i_syms);
-    sh.lens = tb.at<uint8_t>(i_lens);
-    sh.n_syms = (uint32_t)syms.size();
-    sh.n_tables = (uint32_t)(lim.size() / 17);
-    sh.bb = ar.get<uint32_t>(B_all);
-    if (payload_dev)  // the update is in device memory: its block table precedes the payload there
-        HIP_OK(hipMemcpyAsync(sh.bb, payload_dev - (u.payload_offset - u.block_table_offset), 4 * B_all,
-                              hipMemcpyDeviceToDevice, s));
-    else
-        HIP_OK(hipMemcpyAsync(sh.bb, u.block_table, 4 * B_all, hipMemcpyHostToDevice, s));
-    // A device-resident payload is read in place, in the 8-byte aligned words that hold it, when those
-    // words lie inside the allocation the update is in (the first one does: the update's header precedes
-    // the payload; the last one may reach past the update's end).  Otherwise, and from the host, it is
-    // copied into words of its own, zero-padded.
-    bool in_place = false;
-    if (payload_dev && u.payload_len) {
-        const uintptr_t at = reinterpret_cast<uintptr_t>(payload_dev), lead = at & 7;
-        const uint64_t words = (lead + u.payload_len + 7) / 8;
-        hipDeviceptr_t base = nullptr;
-        size_t size = 0;
-        if (hipMemGetAddressRange(&base, &size, reinterpret_cast<hipDeviceptr_t>(at)) == hipSuccess &&
-            at - lead >= reinterpret_cast<uintptr_t>(base) &&
-            at - lead + 8 * words <= reinterpret_cast<uintptr_t>(base) + size) {
-            in_place = true;
-            sh.pay = reinterpret_cast<const uint64_t *>(at - lead);
-            sh.bit0 = 8 * (uint32_t)lead;
-            sh.pay_words = words;
+    const bool small = !payload_dev && 4 * B_all + u.payload_len <= kSmallUpdate;
+    const uint64_t pad_words = (u.payload_len + 7) / 8 + 2;  // a copied payload's words, zero-padded by two
+    const size_t i_bb = small ? tb.add(static_cast<const uint8_t *>(u.block_table), 4 * B_all) : 0,
+                 i_pay = small ? tb.add_padded(u.payload_host, u.payload_len, 8 * pad_words) : 0;
+    auto uploaded = [&] {
+        sh.lim = tb.at<uint32_t>(i_lim);
+        sh.off = tb.at<uint32_t>(i_off);
+        sh.syms = tb.at<uint32_t>(i_syms);
+        sh.lens = tb.at<uint8_t>(i_lens);
+        sh.n_syms = (uint32_t)syms.size();
+        sh.n_tables = (uint32_t)(lim.size() / 17);
+        if (small) {
+            sh.bb = tb.at<uint32_t>(i_bb);
+            sh.pay = tb.at<uint64_t>(i_pay);
+            sh.pay_words = pad_words;
         } else {
-            (void)hipGetLastError();  // an address the runtime does not know: copied instead
-        }
-    }
-    if (!in_place) {
-        sh.pay_words = (u.payload_len + 7) / 8 + 2;
-        uint64_t *pay = ar.get<uint64_t>(sh.pay_words);
-        // the copy fills whole words up to payload_len / 8; the rest (partial last word, two pad words) is zeroed
-        zero(pay + u.payload_len / 8, sh.pay_words - u.payload_len / 8, s);
-        if (u.payload_len) {
-            if (payload_dev)
-                HIP_OK(hipMemcpyAsync(pay, payload_dev, u.payload_len, hipMemcpyDeviceToDevice, s));
+            sh.bb = ar.get<uint32_t>(B_all);
+            if (payload_dev)  // the update is in device memory: its block table precedes the payload there
+                HIP_OK(hipMemcpyAsync(sh.bb, payload_dev - (u.payload_offset - u.block_table_offset), 4 * B_all,
+                                      hipMemcpyDeviceToDevice, s));
             else
-                copy_from_host(reinterpret_cast<uint8_t *>(pay), u.payload_host, u.payload_len, s);
+                HIP_OK(hipMemcpyAsync(sh.bb, u.block_table, 4 * B_all, hipMemcpyHostToDevice, s));
         }
-        sh.pay = pay;
-    }
-    sh.boff = ar.get<unsigned long long>(B_all + 1);
-    launch_scan_u32(sh.bb, B_all, sh.boff, ar.get<unsigned long long>(scan_parts(B_all)), s);
+        // A device-resident payload is read in place, in the 8-byte aligned words that hold it, when those
+        // words lie inside the allocation the update is in (the first one does: the update's header precedes
+        // the payload; the last one may reach past the update's end).  Otherwise, and from the host, it is
+        // copied into words of its own, zero-padded.
+        bool in_place = small;
+        if (payload_dev && u.payload_len) {
+            const uintptr_t at = reinterpret_cast<uintptr_t>(payload_dev), lead = at & 7;
+            const uint64_t words = (lead + u.payload_len + 7) / 8;
+            hipDeviceptr_t base = nullptr;
+            size_t size = 0;
+            if (hipMemGetAddressRange(&base, &size, reinterpret_cast<hipDeviceptr_t>(at)) == hipSuccess &&
+                at - lead >= reinterpret_cast<uintptr_t>(base) &&
+                at - lead + 8 * words <= reinterpret_cast<uintptr_t>(base) + size) {
+                in_place = true;
+                sh.pay = reinterpret_cast<const uint64_t *>(at - lead);
+                sh.bit0 = 8 * (uint32_t)lead;
+                sh.pay_words = words;
+            } else {
+                (void)hipGetLastError();  // an address the runtime does not know: copied instead
+            }
+        }
+        if (!in_place) {
+            sh.pay_words = pad_words;
+            uint64_t *pay = ar.get<uint64_t>(sh.pay_words);
+            // the copy fills whole words up to payload_len / 8; the rest (partial last word, two pad words) is zeroed
+            zero(pay + u.payload_len / 8, sh.pay_words - u.payload_len / 8, s);
+            if (u.payload_len) {
+                if (payload_dev)
+                    HIP_OK(hipMemcpyAsync(pay, payload_dev, u.payload_len, hipMemcpyDeviceToDevice, s));
+                else
+                    copy_from_host(reinterpret_cast<uint8_t *>(pay), u.payload_host, u.payload_len, s);
+            }
+            sh.pay = pay;
+        }
+        sh.boff = ar.get<unsigned long long>(B_all + 1);
+        launch_scan_u32(sh.bb, B_all, sh.boff, ar.get<unsigned long long>(scan_parts(B_all)), s);
+    };
 
     if (!split) {
-        const PartCheck r = apply_part(u, L, parts[0], sh, has_cache, cache_vals, slab, slab_req, false, s, ar, hc);
+        const PartCheck r =
+            apply_part(u, L, parts[0], sh, tb, uploaded, has_cache, cache_vals, slab, slab_req, false, s, ar, hc);
         raise_verdict(u, r.bad, r.delta, r.full, has_cache, cache_vals);
         g_apply_hint.put(hint_key, ar.total);
         // the verdict is final, and the writes behind it are done (the downloads above followed them)
@@ -1622,10 +1678,14 @@ void apply(const Update &u, const uint8_t *payload_dev, uint16_t *const *targets
     unsigned int bad = 0;
     std::vector<uint64_t> delta(T, 0), full(T, 0);
     std::vector<Layout> layouts;
+    tb.commit(ar, s);
+    uploaded();
     for (const ApplyPart &P : parts) layouts.push_back(sub_layout(L, P.t0, P.t1, slab));
     for (size_t k = 0; k < parts.size(); ++k) {
         ar.begin_scope();
-        const PartCheck r = apply_part(u, layouts[k], parts[k], sh, has_cache, cache_vals, slab, slab_req, true, s, ar, hc);
+        UploadBatch ub;
+        const PartCheck r = apply_part(u, layouts[k], parts[k], sh, ub, [] {}, has_cache, cache_vals, slab, slab_req,
+                                       true, s, ar, hc);
         ar.end_scope();
         bad |= r.bad;
         std::copy(r.delta.begin(), r.delta.end(), delta.begin() + parts[k].t0);
@@ -1636,7 +1696,9 @@ void apply(const Update &u, const uint8_t *payload_dev, uint16_t *const *targets
         ar.begin_scope();
         PartCheck r;
         try {
-            r = apply_part(u, layouts[k], parts[k], sh, has_cache, cache_vals, slab, slab_req, false, s, ar, hc);
+            UploadBatch ub;
+            r = apply_part(u, layouts[k], parts[k], sh, ub, [] {}, has_cache, cache_vals, slab, slab_req, false, s, ar,
+                           hc);
         } catch (const std::bad_alloc &) {
             if (!k) throw;  // nothing written yet
             throw DeviceError("out of memory while writing a part of the update; the parts before it are written");
@@ -1917,6 +1979,10 @@ int32_t crx_encoded_write(const crx_encoded *e, const char *const *names, const 
         if (dst_on_device) {
             if (e->n_blocks) HIP_OK(hipMemcpyAsync(dst + off_bt, e->d_block_bits, 4 * e->n_blocks, from_dev, s));
             if (e->payload_len) HIP_OK(hipMemcpyAsync(dst + off_pay, e->d_payload, e->payload_len, from_dev, s));
+        } else if (4 * e->n_blocks + e->payload_len <= kChunk) {  // small: both through pinned memory, one wait
+            d2h(dst + off_bt, reinterpret_cast<const uint8_t *>(e->d_block_bits), 4 * e->n_blocks, s);
+            d2h(dst + off_pay, e->d_payload, e->payload_len, s);
+            sync(s);
         } else {
             HIP_OK(hipStreamSynchronize(s));  // the encode's work, before the staged copies below
             copy_to_host(dst + off_bt, reinterpret_cast<const uint8_t *>(e->d_block_bits), 4 * e->n_blocks, s);

@@ -118,8 +118,10 @@ struct CodeArgs {
     uint32_t *words;                // payload as big-endian bytes in 32-bit words
     unsigned long long *bstart;     // [blocks + 1] bit offset of each block
     uint64_t n_words;               // words allocated: a workgroup whose bits end past them writes nothing
-    unsigned int *overflow;         // |= 2 when that happens
+    unsigned int *overflow;         // cleared by k_code_lengths; |= 2 when that happens
     uint64_t bit_base;              // payload bit of these changes' first bit (a part of a chunked update)
+    uint64_t n_blocks;              // bstart[n_blocks] receives the end of the last block
+    uint64_t n_clear;               // payload words that k_code_lengths clears (it clears *overflow too)
 };
 
 constexpr uint32_t kPeekBits = 10, kPeekLens = 1u << kPeekBits;
@@ -219,39 +221,58 @@ void launch_hist(const HistArgs &a, uint32_t n, hipStream_t s);
 // Per-tensor exclusive scans over slabs of per-slab exponent tables, in place; slabs of tensors with
 // cached counts (descs: hist_in and not cold) are read from those counts.  n_tabs (1 or 2) tables of
 // the same layout are scanned by the same launches, each with its own chunk sums and totals.
+// The plan says how: columns of whole tensors in one launch (cols not null), or chunks of slabs in three.
+constexpr uint32_t kScanThreads = 1024, kScanFewCols = 16;
+constexpr uint32_t kScanTensorTiles = 2048, kScanFewTiles = 128;  // slabs per tensor for 16 columns; for all 256
+struct ScanCols {                   // columns [first, first + n) of a tensor's table
+    uint32_t tensor, first, n, pad;
+};
+struct ScanPlan {
+    const ScanCols *cols = nullptr;
+    uint32_t n_cols = 0;
+    const ScanChunk *chunks = nullptr;
+    const uint32_t *tcb = nullptr;  // [tensors + 1] first chunk of each tensor
+    uint32_t n_chunks = 0;
+};
 struct ScanTabs {
     uint32_t *h[2];       // [tiles][256] tables, scanned in place
     uint32_t *csum[2];    // [chunks][256] chunk sums of each
     uint32_t *totals[2];  // [tensors][256] totals of each
 };
-void launch_scan_tables(const TensorDesc *descs, const ScanTabs &p, uint32_t n_tabs, const ScanChunk *chunks,
-                        uint32_t n_chunks, const uint32_t *tensor_chunk_begin, uint32_t n_tensors, hipStream_t s);
+void launch_scan_tables(const TensorDesc *descs, const ScanTabs &p, uint32_t n_tabs, const ScanPlan &plan,
+                        uint32_t n_tensors, hipStream_t s);
+// result (pinned host memory): groups, changes, *overflow
 void launch_enc_groups(const uint32_t *totals_chg, uint32_t n_tensors, GroupDev *groups, uint32_t *gbase,
-                       unsigned long long *counters, hipStream_t s);
+                       const unsigned int *overflow, unsigned long long *result, hipStream_t s);
 void launch_place(const EncRankArgs &a, uint32_t tiles, const uint32_t *tile_tensor,
                   const uint32_t *hall_pre, const uint32_t *hchg_pre, const uint32_t *gbase,
                   uint64_t *sorted, uint64_t n_sorted, hipStream_t s);
-void launch_r0(GroupDev *groups, uint32_t n_groups, const uint64_t *sorted, hipStream_t s);
 void launch_stats(const StatsArgs &a, hipStream_t s);
 void launch_code_lengths(const CodeArgs &a, hipStream_t s);
-// cmap[c] = group of change kElemsPerThread * c; bmap[b] = group of block b
-void launch_chunk_map(const GroupDev *groups, uint32_t n_groups, uint32_t *cmap, hipStream_t s);
+// cmap[c] = group of change kElemsPerThread * c; with `sorted`, the groups' r0 (and the groups in copy[],
+// unless null); clear[0, n_clear) = 0
+void launch_enc_prep(GroupDev *groups, uint32_t n_groups, const uint64_t *sorted, uint32_t *cmap, GroupDev *copy,
+                     uint32_t *clear, uint32_t n_clear, hipStream_t s);
+// bmap[b] = group of block b, binfo[b]
 void launch_block_map(const GroupDev *groups, uint32_t n_groups, uint32_t *bmap, BlockInfo *binfo, hipStream_t s);
 void launch_pack(const CodeArgs &a, hipStream_t s);
 void launch_block_bits(const unsigned long long *bstart, uint64_t n_blocks, uint32_t *out, unsigned int *overflow,
                        hipStream_t s);
-// Exclusive prefix sums with out[n] = total; `part` holds scan_parts(n) values of scratch.
+// Exclusive prefix sums with out[n] = total; `part` holds scan_parts(n) values of scratch.  Up to
+// kScanOneMax elements: one workgroup, one launch.
+constexpr uint64_t kScanOneMax = 32768;
 uint64_t scan_parts(uint64_t n);
 void launch_scan_u64(const unsigned long long *in, uint64_t n, unsigned long long *out, unsigned long long *part,
                      hipStream_t s);
 void launch_scan_u32(const uint32_t *in, uint64_t n, unsigned long long *out, unsigned long long *part, hipStream_t s);
 // ok = 1 iff *bad is 0 and every tensor's old checksum (cached[t] where has[t], else full[t]) plus
-// its delta equals want[t]; 0 otherwise.  One workgroup.
+// its delta equals want[t]; 0 otherwise.  result (pinned host memory): *bad, delta[n], full[n].  One workgroup.
 void launch_verdict(uint32_t n, const unsigned long long *delta, const uint64_t *full, const int32_t *has,
                     const uint64_t *cached, const uint64_t *want, const unsigned int *bad, unsigned int *ok,
-                    hipStream_t s);
-void launch_tensor_sums(const TensorDesc *descs, uint32_t n_tensors, const uint64_t *per_tile, uint64_t *out,
-                        hipStream_t s);
+                    unsigned long long *result, hipStream_t s);
+// out_a, out_b [tensors]: sums of a and b [tiles] over each tensor's slabs
+void launch_tensor_sums(const TensorDesc *descs, uint32_t n_tensors, const uint64_t *a, const uint64_t *b,
+                        uint64_t *out_a, uint64_t *out_b, hipStream_t s);
 void launch_decode(const DecodeArgs &a, hipStream_t s);
 constexpr uint64_t kDecWaveBlocks = 12288;  // updates of up to so many blocks: a wavefront per block
 constexpr uint32_t kDecSyms = 2048;  // decoding symbols staged in LDS when they fit (with the first indices)

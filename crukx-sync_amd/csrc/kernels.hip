@@ -73,14 +73,6 @@ __global__ __launch_bounds__(256) void k_tile_map(const TensorDesc *descs, uint3
     for (uint32_t i = threadIdx.x; i < d.n_tiles; i += 256) tile_tensor[d.tile_begin + i] = blockIdx.x;
 }
 
-// One workgroup per group: the group of every kElemsPerThread-th change and of every block.
-__global__ __launch_bounds__(256) void k_chunk_map(const GroupDev *groups, uint32_t *cmap) {
-    const GroupDev g = groups[blockIdx.x];
-    const uint64_t c0 = ((uint64_t)g.elem_base + kElemsPerThread - 1) / kElemsPerThread;
-    const uint64_t c1 = ((uint64_t)g.elem_base + g.count + kElemsPerThread - 1) / kElemsPerThread;
-    for (uint64_t c = c0 + threadIdx.x; c < c1; c += 256) cmap[c] = blockIdx.x;
-}
-
 __global__ __launch_bounds__(256) void k_block_map(const GroupDev *groups, uint32_t *bmap, BlockInfo *binfo) {
     const GroupDev g = groups[blockIdx.x];
     const uint32_t nb = (g.count + 255) / 256;
@@ -545,6 +537,48 @@ __global__ __launch_bounds__(256) void k_scan_fin(const TensorDesc *descs, ScanT
     scan_column(src, dst, c.tile_begin, c.tile_end - c.tile_begin, k, p.csum[tab][(uint64_t)i * 256 + k]);
 }
 
+// The same scan in one launch, for tensors of up to kScanTensorTiles slabs: a workgroup takes some columns
+// of one tensor's table (all 256 of a small tensor, 16 of a large one: ScanCols), its threads runs of
+// consecutive slabs of them.  Each thread sums its run, the runs' totals meet in LDS, and each writes its
+// run from the total of those before it.  A run stays in registers, so the table is read once.
+constexpr uint32_t kScanKeep = 32;  // slabs per run
+static_assert(kScanThreads / kScanFewCols * kScanKeep == kScanTensorTiles, "the largest tensor's runs");
+static_assert(kScanThreads / 256 * kScanKeep == kScanFewTiles, "the largest small tensor's runs");
+__global__ __launch_bounds__(kScanThreads) void k_scan_tensor(const TensorDesc *descs, ScanTabs p, const ScanCols *cols,
+                                                              uint32_t n_cols) {
+    __shared__ uint32_t part[kScanThreads];
+    const uint32_t tab = blockIdx.x >= n_cols;
+    const ScanCols sc = cols[blockIdx.x - tab * n_cols];
+    const TensorDesc td = descs[sc.tensor];
+    uint32_t *const h = p.h[tab];
+    const uint32_t c = threadIdx.x & (sc.n - 1), k = sc.first + c, run = threadIdx.x / sc.n, runs = kScanThreads / sc.n;
+    const uint32_t per = (td.n_tiles + runs - 1) / runs;
+    const uint32_t r0 = min(run * per, td.n_tiles), r1 = min(r0 + per, td.n_tiles);
+    // raw buffers over the tensor's table: a row past the run gets an offset past the end, which loads 0
+    // and drops the store
+    const uint32_t bytes = td.n_tiles * 1024u;
+    const Rsrc src = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t *>(scan_src(td, h, td.tile_begin)), (short)0,
+                                                       (int)bytes, 0x00020000);
+    const Rsrc dst = __builtin_amdgcn_make_buffer_rsrc(h + (uint64_t)td.tile_begin * 256, (short)0, (int)bytes, 0x00020000);
+    const uint32_t at = r0 * 1024u + 4 * k, end = r1 * 1024u;
+    auto row = [&](uint32_t j) { return at + j * 1024u < end ? at + j * 1024u : ~0u; };
+    uint32_t x[kScanKeep], s = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kScanKeep; ++j) x[j] = __builtin_amdgcn_raw_buffer_load_b32(src, row(j), 0, 0);
+#pragma unroll
+    for (uint32_t j = 0; j < kScanKeep; ++j) s += x[j];
+    part[threadIdx.x] = s;
+    __syncthreads();
+    uint32_t before = 0;
+    for (uint32_t q = 0; q < run; ++q) before += part[q * sc.n + c];
+    if (run + 1 == runs) p.totals[tab][(uint64_t)sc.tensor * 256 + k] = before + s;
+#pragma unroll
+    for (uint32_t j = 0; j < kScanKeep; ++j) {
+        __builtin_amdgcn_raw_buffer_store_b32(before, dst, row(j), 0, 0);
+        before += x[j];
+    }
+}
+
 // ================================================================== encode: groups and placement
 // Groups are the non-empty (tensor, exponent) pairs in (tensor, exponent) order (codec.py:317-333).
 
@@ -593,16 +627,26 @@ __global__ __launch_bounds__(64) void k_place(EncRankArgs a, const uint32_t *til
     }
 }
 
-// r0 = floor(log2(max(mean gap, 1))) clamped to 30; the gaps of a group sum to last index + 1 - count.
-__global__ __launch_bounds__(256) void k_r0(GroupDev *groups, uint32_t n_groups, const uint64_t *sorted) {
-    const uint32_t g = blockIdx.x * 256 + threadIdx.x;
-    if (g >= n_groups) return;
-    const GroupDev gr = groups[g];
-    const uint64_t last = (uint32_t)sorted[(uint64_t)gr.elem_base + gr.count - 1];
-    const uint64_t s = last + 1 - gr.count;
+// One workgroup per group: the group of every kElemsPerThread-th change (cmap), and the group with its
+// r0 = floor(log2(max(mean gap, 1))) clamped to 30 (the gaps of a group sum to last index + 1 - count;
+// `sorted` null: r0 stays), in place and, with `copy`, to copy[g]; the workgroups together clear
+// clear[0, n_clear).  Launch-bound at small sizes: as three launches (a map, r0, a fill) it took 4-10 us
+// more per encode.
+__global__ __launch_bounds__(256) void k_enc_prep(GroupDev *groups, const uint64_t *sorted, uint32_t *cmap,
+                                                  GroupDev *copy, uint32_t *clear, uint32_t n_clear) {
+    GroupDev g = groups[blockIdx.x];
+    const uint64_t c0 = ((uint64_t)g.elem_base + kElemsPerThread - 1) / kElemsPerThread;
+    const uint64_t c1 = ((uint64_t)g.elem_base + g.count + kElemsPerThread - 1) / kElemsPerThread;
+    for (uint64_t c = c0 + threadIdx.x; c < c1; c += 256) cmap[c] = blockIdx.x;
+    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n_clear; i += (uint64_t)gridDim.x * 256) clear[i] = 0;
+    if (threadIdx.x || !sorted) return;
+    const uint64_t last = (uint32_t)sorted[(uint64_t)g.elem_base + g.count - 1];
+    const uint64_t s = last + 1 - g.count;
     uint32_t r0 = 0;
-    while (r0 < 30 && ((uint64_t)gr.count << (r0 + 1)) <= s) ++r0;
-    groups[g].r0 = r0;
+    while (r0 < 30 && ((uint64_t)g.count << (r0 + 1)) <= s) ++r0;
+    g.r0 = r0;
+    groups[blockIdx.x] = g;
+    if (copy) copy[blockIdx.x] = g;
 }
 
 // Records of a workgroup's changes in LDS: thread t's kElemsPerThread records at t * kRecPad (the pad
@@ -815,11 +859,12 @@ __device__ unsigned long long block_exclusive_sum(unsigned long long v, unsigned
 
 // Groups from the (tensor, exponent) change totals, in that order: kGroupChunk totals per workgroup
 // (16 consecutive per thread).  A workgroup first sums the totals before its chunk (coalesced, a few
-// hundred KB at most), then scans its own.  gbase[i] = changes before entry i; counters[0] = groups,
-// counters[1] = changes (written by the last workgroup).
+// hundred KB at most), then scans its own.  gbase[i] = changes before entry i.  The last workgroup writes
+// result[0] = groups, result[1] = changes, result[2] = *overflow into pinned host memory.
 constexpr uint32_t kGroupChunk = 4096;
 __global__ __launch_bounds__(256) void k_enc_groups(const uint32_t *tot, uint32_t n_tensors, GroupDev *groups,
-                                                    uint32_t *gbase, unsigned long long *counters) {
+                                                    uint32_t *gbase, const unsigned int *overflow,
+                                                    unsigned long long *result) {
     __shared__ unsigned long long sh[8];
     const uint32_t tid = threadIdx.x;
     const uint64_t n = (uint64_t)n_tensors * 256, c0 = (uint64_t)blockIdx.x * kGroupChunk;
@@ -867,14 +912,18 @@ __global__ __launch_bounds__(256) void k_enc_groups(const uint32_t *tot, uint32_
         }
     }
     if (blockIdx.x + 1 == gridDim.x && tid == 0) {
-        counters[0] = bz + tz;  // groups
-        counters[1] = bv + tv;  // changes
+        result[0] = bz + tz;  // groups
+        result[1] = bv + tv;  // changes
+        result[2] = *overflow;
     }
 }
 
 __global__ __launch_bounds__(256) void k_code_lengths(CodeArgs a) {
     __shared__ uint64_t rec[256 * kRecPad];
     const uint64_t wbase = (uint64_t)blockIdx.x * kElemsPerWG;
+    // the payload's words, for k_pack: cleared here, where there is memory bandwidth to spare
+    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < a.n_clear; i += (uint64_t)gridDim.x * 256) a.words[i] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *a.overflow = 0;
     stage_records(a.sorted, a.n, wbase, rec);
     ThreadCodes tc;
     thread_codes(a, rec, wbase, tc);
@@ -965,6 +1014,8 @@ __device__ __forceinline__ void pack_thread(const CodeArgs &a, const ThreadCodes
         }
     }
     bw.finish();
+    // the end of the last block
+    if (tc.n && (uint64_t)(blockIdx.x * 256ull + threadIdx.x) * kElemsPerThread + tc.n == a.n) a.bstart[a.n_blocks] = off;
 }
 
 // The workgroup's bits are assembled in LDS (the record staging area, free once the codes are in
@@ -1074,16 +1125,65 @@ __global__ __launch_bounds__(256) void k_scan_down(const T *in, uint64_t n, cons
     if (blockIdx.x == gridDim.x - 1 && tid == 0) out[n] = part[gridDim.x];
 }
 
+// The same scan of up to a few ten thousand elements by one workgroup, in one launch: 16 consecutive
+// elements per thread, kScanOneChunk per round.
+constexpr uint32_t kScanOneThreads = 1024, kScanOneChunk = 16 * kScanOneThreads;
+template <typename T>
+__global__ __launch_bounds__(kScanOneThreads) void k_scan_one(const T *in, uint32_t n, unsigned long long *out) {
+    __shared__ unsigned long long sh[kScanOneThreads / 64];
+    const uint32_t ln = lane(), w = threadIdx.x >> 6;
+    unsigned long long carry = 0;
+    for (uint32_t b = 0; b < n; b += kScanOneChunk) {
+        const uint32_t i0 = b + 16 * threadIdx.x;
+        unsigned long long v[16], s = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < 16; ++k) v[k] = i0 + k < n ? (unsigned long long)in[i0 + k] : 0ULL;
+#pragma unroll
+        for (uint32_t k = 0; k < 16; ++k) s += v[k];
+        unsigned long long incl = s;
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned long long t = __shfl_up(incl, o, 64);
+            if (ln >= (uint32_t)o) incl += t;
+        }
+        if (ln == 63) sh[w] = incl;
+        __syncthreads();
+        unsigned long long run = carry + incl - s, tot = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < kScanOneThreads / 64; ++q) {
+            const unsigned long long x = sh[q];
+            run += q < w ? x : 0ULL;
+            tot += x;
+        }
+        __syncthreads();  // sh is written again in the next round
+#pragma unroll
+        for (uint32_t k = 0; k < 16; ++k) {
+            if (i0 + k < n) out[i0 + k] = run;
+            run += v[k];
+        }
+        carry += tot;
+    }
+    if (threadIdx.x == 0) out[n] = carry;
+}
+
 __global__ void k_scan_empty(unsigned long long *out) { out[0] = 0; }
 
-__global__ __launch_bounds__(256) void k_tensor_sums(const TensorDesc *descs, const uint64_t *per_tile, uint64_t *out) {
-    __shared__ unsigned long long sh[256];
+// One workgroup per tensor: the sums of two per-slab arrays over its slabs.
+__global__ __launch_bounds__(256) void k_tensor_sums(const TensorDesc *descs, const uint64_t *a, const uint64_t *b,
+                                                     uint64_t *out_a, uint64_t *out_b) {
+    __shared__ unsigned long long sh[4];
     const TensorDesc td = descs[blockIdx.x];
-    unsigned long long s = 0;
-    for (uint32_t t = threadIdx.x; t < td.n_tiles; t += 256) s += per_tile[td.tile_begin + t];
-    unsigned long long total;
-    block_exclusive_sum(s, sh, &total);
-    if (threadIdx.x == 0) out[blockIdx.x] = total;
+    unsigned long long sa = 0, sb = 0;
+    for (uint32_t t = threadIdx.x; t < td.n_tiles; t += 256) {
+        sa += a[td.tile_begin + t];
+        sb += b[td.tile_begin + t];
+    }
+    unsigned long long ta, tb;
+    block_exclusive_sum(sa, sh, &ta);
+    block_exclusive_sum(sb, sh, &tb);
+    if (threadIdx.x == 0) {
+        out_a[blockIdx.x] = ta;
+        out_b[blockIdx.x] = tb;
+    }
 }
 
 // Full checksum of one tensor: each workgroup sums a contiguous range into partial[blockIdx.x].
@@ -2349,19 +2449,27 @@ __global__ __launch_bounds__(256) void k_verify(SlabArgs a) {
 }
 
 // The host's verdict (codec.py:598-604,696-712), computed on the device as well so that the scatter
-// can follow it without a host round trip; the host still raises the errors from the same data.
+// can follow it without a host round trip; the host still raises the errors from the same data, which
+// the kernel writes into pinned host memory: result[0] = *bad, then the deltas, then the full sums (three
+// copies behind the commit took 10 us each).
 __global__ __launch_bounds__(256) void k_verdict(uint32_t n, const unsigned long long *delta, const uint64_t *full,
                                                  const int32_t *has, const uint64_t *cached, const uint64_t *want,
-                                                 const unsigned int *bad, unsigned int *ok) {
+                                                 const unsigned int *bad, unsigned int *ok, unsigned long long *result) {
     __shared__ unsigned int miss;
     if (threadIdx.x == 0) miss = 0;
     __syncthreads();
     for (uint32_t t = threadIdx.x; t < n; t += 256) {
-        const uint64_t old = has[t] ? cached[t] : full[t];
-        if (old + delta[t] != want[t]) atomicOr(&miss, 1u);
+        const uint64_t d = delta[t], f = full[t];
+        const uint64_t old = has[t] ? cached[t] : f;
+        if (old + d != want[t]) atomicOr(&miss, 1u);
+        result[1 + t] = d;
+        result[1 + n + t] = f;
     }
     __syncthreads();
-    if (threadIdx.x == 0) *ok = (miss == 0 && *bad == 0) ? 1u : 0u;
+    if (threadIdx.x == 0) {
+        *ok = (miss == 0 && *bad == 0) ? 1u : 0u;
+        result[0] = *bad;
+    }
 }
 
 // After the device's verdict, one workgroup per slab.  A slab with more than one window: its writes,
@@ -2419,17 +2527,27 @@ void launch_enc_rank(const EncRankArgs &a, uint32_t tiles, hipStream_t s) {
 }
 void launch_hist(const HistArgs &a, uint32_t n, hipStream_t s) { CRX_LAUNCH("apply_hist", k_hist, n, 64, s, a); }
 
-void launch_scan_tables(const TensorDesc *descs, const ScanTabs &p, uint32_t n_tabs, const ScanChunk *chunks,
-                        uint32_t n_chunks, const uint32_t *tensor_chunk_begin, uint32_t n_tensors, hipStream_t s) {
+// One launch while every tensor's runs fit a workgroup's registers; else the chunked three, which spread
+// a tensor over as many workgroups as it has chunks.  Measured (two tables, encode): 200,000 weights in
+// 390 slabs 12 us, in three launches 19; 26.6M weights in 3250 slabs 14 against 21.
+void launch_scan_tables(const TensorDesc *descs, const ScanTabs &p, uint32_t n_tabs, const ScanPlan &plan,
+                        uint32_t n_tensors, hipStream_t s) {
+    if (plan.cols) {
+        CRX_LAUNCH("scan_tensor", k_scan_tensor, n_tabs * plan.n_cols, kScanThreads, s, descs, p, plan.cols, plan.n_cols);
+        return;
+    }
+    const uint32_t n_chunks = plan.n_chunks;
+    const ScanChunk *const chunks = plan.chunks;
+    const uint32_t *const tensor_chunk_begin = plan.tcb;
     CRX_LAUNCH("scan_sum", k_scan_sum, n_tabs * n_chunks, 256, s, descs, p, chunks, n_chunks);
     CRX_LAUNCH("scan_mid", k_scan_mid, n_tabs * n_tensors, 256, s, p, tensor_chunk_begin, n_tensors);
     CRX_LAUNCH("scan_fin", k_scan_fin, n_tabs * n_chunks, 256, s, descs, p, chunks, n_chunks);
 }
 
 void launch_enc_groups(const uint32_t *totals_chg, uint32_t n_tensors, GroupDev *groups, uint32_t *gbase,
-                       unsigned long long *counters, hipStream_t s) {
+                       const unsigned int *overflow, unsigned long long *result, hipStream_t s) {
     CRX_LAUNCH("enc_groups", k_enc_groups, grid1((uint64_t)n_tensors * 256, kGroupChunk), 256, s, totals_chg, n_tensors,
-               groups, gbase, counters);
+               groups, gbase, overflow, result);
 }
 
 void launch_place(const EncRankArgs &a, uint32_t tiles, const uint32_t *tile_tensor, const uint32_t *hall_pre,
@@ -2441,14 +2559,11 @@ void launch_tile_map(const TensorDesc *descs, uint32_t n_tensors, uint32_t *tile
     CRX_LAUNCH("tile_map", k_tile_map, n_tensors, 256, s, descs, tile_tensor);
 }
 
-void launch_r0(GroupDev *groups, uint32_t n_groups, const uint64_t *sorted, hipStream_t s) {
-    CRX_LAUNCH("rice_r0", k_r0, grid1(n_groups, 256), 256, s, groups, n_groups, sorted);
-}
-
 void launch_stats(const StatsArgs &a, hipStream_t s) { CRX_LAUNCH("stats", k_stats, grid1(a.n, kElemsPerWG), 256, s, a); }
 
-void launch_chunk_map(const GroupDev *groups, uint32_t n_groups, uint32_t *cmap, hipStream_t s) {
-    CRX_LAUNCH("chunk_map", k_chunk_map, n_groups, 256, s, groups, cmap);
+void launch_enc_prep(GroupDev *groups, uint32_t n_groups, const uint64_t *sorted, uint32_t *cmap, GroupDev *copy,
+                     uint32_t *clear, uint32_t n_clear, hipStream_t s) {
+    CRX_LAUNCH("enc_prep", k_enc_prep, n_groups, 256, s, groups, sorted, cmap, copy, clear, n_clear);
 }
 
 void launch_block_map(const GroupDev *groups, uint32_t n_groups, uint32_t *bmap, BlockInfo *binfo, hipStream_t s) {
@@ -2475,6 +2590,10 @@ static void launch_scan(const char *name, const T *in, uint64_t n, unsigned long
         CRX_LAUNCH(name, k_scan_empty, 1, 1, s, out);
         return;
     }
+    if (n <= kScanOneMax) {
+        CRX_LAUNCH(name, k_scan_one<T>, 1, kScanOneThreads, s, in, (uint32_t)n, out);
+        return;
+    }
     const uint64_t m = (n + kScanChunk - 1) / kScanChunk;
     CRX_LAUNCH(name, k_scan_reduce<T>, (uint32_t)m, 256, s, in, n, part);
     CRX_LAUNCH(name, k_scan_parts, 1, 256, s, part, m);
@@ -2492,15 +2611,13 @@ void launch_scan_u32(const uint32_t *in, uint64_t n, unsigned long long *out, un
 
 void launch_verdict(uint32_t n, const unsigned long long *delta, const uint64_t *full, const int32_t *has,
                     const uint64_t *cached, const uint64_t *want, const unsigned int *bad, unsigned int *ok,
-                    hipStream_t s) {
-    timing_begin("verdict", s);
-    hipLaunchKernelGGL(k_verdict, dim3(1), dim3(256), 0, s, n, delta, full, has, cached, want, bad, ok);
-    timing_end("verdict", s);
+                    unsigned long long *result, hipStream_t s) {
+    CRX_LAUNCH("verdict", k_verdict, 1, 256, s, n, delta, full, has, cached, want, bad, ok, result);
 }
 
-void launch_tensor_sums(const TensorDesc *descs, uint32_t n_tensors, const uint64_t *per_tile, uint64_t *out,
-                        hipStream_t s) {
-    CRX_LAUNCH("tensor_sums", k_tensor_sums, n_tensors, 256, s, descs, per_tile, out);
+void launch_tensor_sums(const TensorDesc *descs, uint32_t n_tensors, const uint64_t *a, const uint64_t *b,
+                        uint64_t *out_a, uint64_t *out_b, hipStream_t s) {
+    CRX_LAUNCH("tensor_sums", k_tensor_sums, n_tensors, 256, s, descs, a, b, out_a, out_b);
 }
 
 void launch_decode(const DecodeArgs &a, hipStream_t s) {
