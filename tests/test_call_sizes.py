@@ -29,7 +29,8 @@ def test_count_slab_follows_the_size():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n", [1, 511, 512, 513, 70_001, 512 * 4096, 512 * 4096 + 1])
+@pytest.mark.parametrize("n", [1, 511, 512, 513, 512 * 128, 512 * 128 + 1, 512 * 2048, 512 * 2048 + 1, 512 * 4096,
+                               512 * 4096 + 1])
 def test_bytes_and_apply_at_slab_edges(n):
     a, b = scenarios.rl_pair(n, lr=4e-6, seed=n)
     b[-1] = (b[-1:].view(torch.int16) + 1).view(torch.bfloat16)[0]  # at least one change, in the last slab
@@ -111,3 +112,34 @@ def test_blocks_of_long_codes(spread):
     recv = _cuda(old)
     crukx_sync.apply_update(recv, upd)
     assert torch.equal(recv["w"].cpu(), b)
+
+
+def _packed(tensors, lead):
+    """The tensors one behind another in one GPU buffer, from element `lead` of it on."""
+    flat = torch.zeros(lead + sum(t.numel() for t in tensors.values()), dtype=torch.int16, device="cuda")
+    out, at = {}, lead
+    for k, t in tensors.items():
+        out[k] = flat[at:at + t.numel()].view(t.dtype).view(t.shape)
+        out[k].copy_(t)
+        at += t.numel()
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("leads", [(0, 0), (1, 1), (0, 1), (1, 0)])
+@pytest.mark.parametrize("cached", [False, True])
+def test_packed_tensors_at_odd_elements(leads, cached):
+    """Old and new state dicts packed into flat buffers, beginning in the same or in different halves of
+    a 32-bit word, with and without the sender's cache: the oracle's bytes, and the inputs unchanged."""
+    old, new = {}, {}
+    for i, n in enumerate([1, 2, 511, 513, 70_001, 1025]):
+        old[f"t{i}"], new[f"t{i}"] = scenarios.rl_pair(n, lr=4e-6, seed=300 + i)
+        new[f"t{i}"][-1] = (new[f"t{i}"][-1:].view(torch.int16) ^ 1).view(torch.bfloat16)[0]
+        new[f"t{i}"][0] = (old[f"t{i}"][:1].view(torch.int16) ^ 3).view(torch.bfloat16)[0]
+    chk = {k: oracle.checksum(t) for k, t in old.items()} if cached else None
+    a, b = _packed(old, leads[0]), _packed(new, leads[1])
+    assert crukx_sync.encode_update(a, b, chk) == oracle.encode_update(old, new)
+    for k in old:
+        assert torch.equal(a[k].cpu().view(torch.int16), old[k].view(torch.int16))
+        assert torch.equal(b[k].cpu().view(torch.int16), new[k].view(torch.int16))
+        assert chk is None or chk[k] == oracle.checksum(new[k])
