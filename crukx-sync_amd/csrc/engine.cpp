@@ -979,6 +979,29 @@ uint64_t build_tables(const std::vector<uint64_t> &dense, const std::vector<std:
     return bits;
 }
 
+// The code kernels' inputs and their own buffers; the payload's are left to the caller.
+CodeArgs code_args(Arena &ar, const uint64_t *sorted, uint64_t n, const GroupDev *groups, uint32_t n_groups,
+                   const uint32_t *lut, const uint32_t *rare_keys, const uint32_t *rare_vals, uint32_t n_rare,
+                   const uint32_t *cmap, uint64_t n_blocks) {
+    const uint64_t n_wg = (n + kElemsPerWG - 1) / kElemsPerWG;
+    CodeArgs ca{};
+    ca.sorted = sorted;
+    ca.n = n;
+    ca.groups = groups;
+    ca.n_groups = n_groups;
+    ca.lut = lut;
+    ca.rare_keys = rare_keys;
+    ca.rare_vals = rare_vals;
+    ca.n_rare = n_rare;
+    ca.cmap = cmap;
+    ca.wbits = ar.get<unsigned long long>(n_wg);
+    ca.stage = ar.get<uint32_t>(n_wg * kStageStride);
+    ca.bstart = ar.get<unsigned long long>(n_blocks + 1);
+    ca.bwg = ar.get<uint32_t>(n_blocks + 1);
+    ca.n_blocks = n_blocks;
+    return ca;
+}
+
 // An update encoded part by part (more changes than one pass indexes in 32 bits, or parts asked for):
 // the tensors in parts of at most `limit` elements.  Pass 1 ranks each part for its groups, symbol
 // counts and checksum parts; the tables are built from the whole update's counts (codec.py:362-392);
@@ -1115,19 +1138,22 @@ void encode_parts(const Layout &L, uint64_t limit, uint32_t slab, const int32_t 
         const uint64_t n_thr = (p.C + kElemsPerThread - 1) / kElemsPerThread;
         uint32_t *cmap = ar.get<uint32_t>(n_thr);
         launch_enc_prep(d_groups, (uint32_t)G, nullptr, cmap, nullptr, nullptr, 0, s);
-        unsigned long long *tsum = ar.get<unsigned long long>(n_thr), *toff = ar.get<unsigned long long>(n_thr + 1);
-        unsigned long long *bstart = ar.get<unsigned long long>(p.B + 1);
         unsigned int *bovf = ar.get<unsigned int>(1);
-        CodeArgs ca{sorted, p.C, d_groups, (uint32_t)G, d_lut, d_rk, d_rv, (uint32_t)rkeys.size(), cmap, tsum, toff,
-                    words, bstart, n_words, bovf, p.bit0, p.B, 0};
-        launch_code_lengths(ca, s);
-        launch_scan_u64(tsum, n_thr, toff, ar.get<unsigned long long>(scan_parts(n_thr)), s);
-        launch_pack(ca, s);
-        launch_block_bits(bstart, p.B, bb + p.blk0, bovf, s);
+        CodeArgs ca = code_args(ar, sorted, p.C, d_groups, (uint32_t)G, d_lut, d_rk, d_rv, (uint32_t)rkeys.size(), cmap, p.B);
+        ca.words = words;
+        ca.n_words = n_words;
+        ca.overflow = bovf;
+        ca.bit_base = p.bit0;
+        const uint64_t n_wg = (p.C + kElemsPerWG - 1) / kElemsPerWG;
+        unsigned long long *woff = ar.get<unsigned long long>(n_wg + 1);
+        ca.woff = woff;
+        launch_code(ca, s);
+        launch_scan_u64(ca.wbits, n_wg, woff, ar.get<unsigned long long>(scan_parts(n_wg)), s);
+        launch_join_bits(ca, bb + p.blk0, s);
         unsigned int hovf = 0;
         unsigned long long dev_bits = 0;
         d2h(&hovf, bovf, 1, s);
-        d2h(&dev_bits, toff + n_thr, 1, s);
+        d2h(&dev_bits, woff + n_wg, 1, s);
         sync(s);
         ar.end_scope();
         if (hovf & 2u || dev_bits != p.bits) throw DeviceError("the packed payload's size differs from its codes' lengths");
@@ -1262,21 +1288,21 @@ void encode(int32_t n, const uint16_t *const *olds, const uint16_t *const *news,
     ub.commit(ar, s);
     GroupDev *d_groups2 = ub.at<GroupDev>(i_groups);
     uint32_t *d_lut = ub.at<uint32_t>(i_lut), *d_rk = ub.at<uint32_t>(i_rk), *d_rv = ub.at<uint32_t>(i_rv);
-    // the bit offsets, their total, and the flags of the code kernels behind it: one copy brings both back
-    unsigned long long *tsum = ar.get<unsigned long long>(n_thr), *toff = ar.get<unsigned long long>(n_thr + 2);
-    unsigned int *bovf = reinterpret_cast<unsigned int *>(toff + n_thr + 1);
-    const uint64_t n_words = (total_bits + 31) / 32 + 4;
-    uint32_t *words = ar.get<uint32_t>(n_words);
-    unsigned long long *bstart = ar.get<unsigned long long>(B + 1);
+    // the workgroups' bit offsets, their total, and the flags of the code kernels behind it: one copy
+    // brings both back
+    const uint64_t n_wg = (C + kElemsPerWG - 1) / kElemsPerWG;
+    unsigned long long *woff = ar.get<unsigned long long>(n_wg + 2);
     uint32_t *bb = ar.get<uint32_t>(B);
-    CodeArgs ca{sorted, C, d_groups2, (uint32_t)G, d_lut, d_rk, d_rv, (uint32_t)rkeys.size(), cmap, tsum, toff,
-                words, bstart, n_words, bovf, 0, B, n_words};
-    launch_code_lengths(ca, s);
-    launch_scan_u64(tsum, n_thr, toff, ar.get<unsigned long long>(scan_parts(n_thr)), s);
-    launch_pack(ca, s);
-    launch_block_bits(bstart, B, bb, bovf, s);
+    CodeArgs ca = code_args(ar, sorted, C, d_groups2, (uint32_t)G, d_lut, d_rk, d_rv, (uint32_t)rkeys.size(), cmap, B);
+    ca.n_words = ca.n_clear = (total_bits + 31) / 32 + 4;
+    uint32_t *words = ca.words = ar.get<uint32_t>(ca.n_words);
+    ca.woff = woff;
+    ca.overflow = reinterpret_cast<unsigned int *>(woff + n_wg + 1);
+    launch_code(ca, s);
+    launch_scan_u64(ca.wbits, n_wg, woff, ar.get<unsigned long long>(scan_parts(n_wg)), s);
+    launch_join_bits(ca, bb, s);
     unsigned long long last[2] = {0, 0};  // the bits of all codes, the flags
-    d2h(last, toff + n_thr, 2, s);
+    d2h(last, woff + n_wg, 2, s);
 
     // the rest of the host's part while the device packs: checksums (codec.py:344-352), the groups
     for (uint32_t d = 0; d < T; ++d) {

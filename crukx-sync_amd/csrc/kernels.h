@@ -13,6 +13,8 @@ constexpr int kLocalGroups = 64;      // groups a statistics workgroup accumulat
 constexpr uint32_t kScanTiles = 32;   // slabs per chunk of the per-tensor histogram scan
 constexpr int kElemsPerThread = 16;   // change-order kernels: contiguous elements per thread
 constexpr int kElemsPerWG = 256 * kElemsPerThread;
+constexpr uint32_t kStageWords = 2048;  // encode: words staged for a workgroup's codes (16 bits per change)
+constexpr uint32_t kStageStride = kStageWords + 4;  // room for a 16-byte load at the last
 constexpr uint32_t kNone = 0xFFFFFFFFu;
 constexpr int32_t kFar = 0x40000000;  // "no target in this slab" for the select pass
 // bits of the apply verdict flag
@@ -113,15 +115,19 @@ struct CodeArgs {
     const uint32_t *rare_vals;
     uint32_t n_rare;
     const uint32_t *cmap;           // [n / kElemsPerThread] group of every thread's first change
-    unsigned long long *tsum;       // [threads] bits per thread (kElemsPerThread changes)
-    const unsigned long long *toff; // [threads] exclusive bit offsets
+    unsigned long long *wbits;      // [workgroups] bits of each workgroup's codes (kElemsPerWG changes)
+    const unsigned long long *woff; // [workgroups + 1] their exclusive sums
+    uint32_t *stage;                // [workgroups][kStageStride] each workgroup's bits
     uint32_t *words;                // payload as big-endian bytes in 32-bit words
-    unsigned long long *bstart;     // [blocks + 1] bit offset of each block
+    // [blocks + 1] first bit of each block (then the end of the last), from the first bit of the codes of
+    // workgroup bwg, in which it begins
+    unsigned long long *bstart;
+    uint32_t *bwg;
     uint64_t n_words;               // words allocated: a workgroup whose bits end past them writes nothing
-    unsigned int *overflow;         // cleared by k_code_lengths; |= 2 when that happens
+    unsigned int *overflow;         // cleared by k_code; |= 2 when that happens, |= 1 for a block of 2^32 bits
     uint64_t bit_base;              // payload bit of these changes' first bit (a part of a chunked update)
-    uint64_t n_blocks;              // bstart[n_blocks] receives the end of the last block
-    uint64_t n_clear;               // payload words that k_code_lengths clears (it clears *overflow too)
+    uint64_t n_blocks;
+    uint64_t n_clear;               // payload words that k_code clears
 };
 
 constexpr uint32_t kPeekBits = 10, kPeekLens = 1u << kPeekBits;
@@ -248,16 +254,16 @@ void launch_place(const EncRankArgs &a, uint32_t tiles, const uint32_t *tile_ten
                   const uint32_t *hall_pre, const uint32_t *hchg_pre, const uint32_t *gbase,
                   uint64_t *sorted, uint64_t n_sorted, hipStream_t s);
 void launch_stats(const StatsArgs &a, hipStream_t s);
-void launch_code_lengths(const CodeArgs &a, hipStream_t s);
+// each workgroup's codes as a bit string of its own and their lengths (wbits); then, with the lengths
+// summed (woff), the strings joined into the payload and the blocks' bits
+void launch_code(const CodeArgs &a, hipStream_t s);
+void launch_join_bits(const CodeArgs &a, uint32_t *block_bits, hipStream_t s);
 // cmap[c] = group of change kElemsPerThread * c; with `sorted`, the groups' r0 (and the groups in copy[],
 // unless null); clear[0, n_clear) = 0
 void launch_enc_prep(GroupDev *groups, uint32_t n_groups, const uint64_t *sorted, uint32_t *cmap, GroupDev *copy,
                      uint32_t *clear, uint32_t n_clear, hipStream_t s);
 // bmap[b] = group of block b, binfo[b]
 void launch_block_map(const GroupDev *groups, uint32_t n_groups, uint32_t *bmap, BlockInfo *binfo, hipStream_t s);
-void launch_pack(const CodeArgs &a, hipStream_t s);
-void launch_block_bits(const unsigned long long *bstart, uint64_t n_blocks, uint32_t *out, unsigned int *overflow,
-                       hipStream_t s);
 // Exclusive prefix sums with out[n] = total; `part` holds scan_parts(n) values of scratch.  Up to
 // kScanOneMax elements: one workgroup, one launch.
 constexpr uint64_t kScanOneMax = 32768;
