@@ -114,6 +114,28 @@ def test_blocks_of_long_codes(spread):
     assert torch.equal(recv["w"].cpu(), b)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("gap", [14, 15, 16, 66, 67, 90])
+def test_workgroups_of_long_bit_strings(gap):
+    """Workgroups of 4096 changes that take gap + 1 bits each (a million changes in one run hold the Rice
+    parameter at 0): as many as are staged at most (16 per change), as are assembled in LDS at most (68),
+    and more."""
+    dense, far = 1 << 20, 3 * 4096 + 17
+    a = torch.full((dense + gap * far,), 0x3F80, dtype=torch.int16)
+    b = a.clone()
+    b[:dense] += 1
+    b[dense::gap] += 1
+    old, new = {"w": a}, {"w": b}
+    upd = crukx_sync.encode_update(_cuda(old), _cuda(new))
+    assert upd == oracle.encode_update(old, new)
+    bits = 8 * _native.lib().crx_update_payload_len(crukx_sync.parse(upd).handle)
+    # the first of the far changes follows the run at once
+    assert 0 <= bits - (2 * dense + 2 + (far - 1) * (gap + 1)) < 8
+    recv = _cuda(old)
+    crukx_sync.apply_update(recv, upd)
+    assert torch.equal(recv["w"].cpu(), b)
+
+
 def _packed(tensors, lead):
     """The tensors one behind another in one GPU buffer, from element `lead` of it on."""
     flat = torch.zeros(lead + sum(t.numel() for t in tensors.values()), dtype=torch.int16, device="cuda")
