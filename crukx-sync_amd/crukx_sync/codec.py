@@ -401,15 +401,17 @@ def _apply_inputs(names, numels, weights, checksums):
             array("Q", [h[0] & _MASK64 if o else 0 for h, o in zip(hits, ok)]), ptrs)
 
 
-def _count_slab(u, usable, numels, slab):
-    """The slab size of an apply of `u` to tensors of `numels` elements, whose usable counts are `usable`
-    (an entry of _hist, or None, per tensor): that of the counts that cover half of the elements, so that
-    a receiver whose updates hold now more, now fewer of its tensors or changes keeps its counts; else the
-    one that suits the update."""
+def _count_slab(u, sizes, numels, slab):
+    """The slab size of an apply of `u` to tensors of `numels` elements, whose usable counts have slabs of
+    `sizes` (0: none; empty: no counts are kept): that of the counts that cover half of the elements, so
+    that a receiver whose updates hold now more, now fewer of its tensors or changes keeps its counts; else
+    the one that suits the update."""
+    if sizes and sizes[0] and sizes.count(sizes[0]) == len(sizes):  # the usual: all of one size
+        return sizes[0]
     elements, by = sum(numels), {}
-    for e, k in zip(usable, numels):
-        if e is not None:
-            by[e[6]] = by.get(e[6], 0) + k
+    for size, k in zip(sizes, numels):
+        if size:
+            by[size] = by.get(size, 0) + k
     for size, k in by.items():
         if 2 * k >= elements:
             return size
@@ -500,7 +502,7 @@ def apply(weights: Mapping[str, torch.Tensor], u: Update, checksums: dict | None
     # exponent counts carried across updates: only for tensors updated in place with a trusted cache
     keep = checksums is not None and staged is targets and _COUNT_CACHE
     slab = int(_SLAB)
-    hist_in, hist_out, bufs, usable = [], [], [], []
+    hist_in, hist_out, bufs, sizes = [], [], [], []
     if keep:
         # an entry is used for the same tensor object, unmodified since, with the same _SLAB and
         # device, when the tensor's checksum is trusted too (one pass over the tensors)
@@ -508,19 +510,23 @@ def apply(weights: Mapping[str, torch.Tensor], u: Update, checksums: dict | None
             hg = _hist.get
             for a, c, v in zip(targets, has, vers):
                 e = hg(id(a)) if c else None
-                ok = e is not None and e[1] == v and e[3] == slab and e[4] == dev and e[0]() is a
-                usable.append(e if ok else None)
-    size = _count_slab(u, usable, numels, slab)
-    if keep:
-        fresh = []
-        for i, e in enumerate(usable):
-            if e is not None and e[6] == size:
-                bufs.append(e[2])
-                hist_in.append(e[5])
-            else:
+                if e is not None:
+                    ref, ver, buf, sl, on, at, k = e
+                    if ver == v and sl == slab and on == dev and ref() is a:
+                        bufs.append(buf)
+                        hist_in.append(at)
+                        sizes.append(k)
+                        continue
                 bufs.append(None)
                 hist_in.append(0)
-                fresh.append(i)
+                sizes.append(0)
+    size = _count_slab(u, sizes, numels, slab)
+    if keep:
+        fresh = []  # tensors without counts of this slab size
+        if sizes.count(size) != len(sizes):
+            fresh = [i for i, k in enumerate(sizes) if k != size]
+            for i in fresh:
+                bufs[i], hist_in[i] = None, 0
         hist_out = list(hist_in)
         # tensors without usable counts: one allocation, sliced per tensor
         fresh = [(i, L.crx_apply_hist_words(targets[i].numel(), size)) for i in fresh]

@@ -1690,8 +1690,17 @@ void apply(const Update &u, const uint8_t *payload_dev, uint16_t *const *targets
     };
 
     if (!split) {
-        const PartCheck r =
-            apply_part(u, L, parts[0], sh, tb, uploaded, has_cache, cache_vals, slab, slab_req, false, s, ar, hc);
+        // A small call's tables travel with the part's other uploads (a copy less: 7-10 us).  In a larger one
+        // they go ahead, so that the device copies and sums the block table while the host prepares the
+        // part (1.5B weights, 1%: 2.42 ms together, 2.39 ahead, with the Python layer's part of the same step).
+        const bool together = small || L.tiles <= kForkTiles;
+        if (!together) {
+            tb.commit(ar, s);
+            uploaded();
+        }
+        UploadBatch ub;
+        const PartCheck r = apply_part(u, L, parts[0], sh, together ? tb : ub, [&] { if (together) uploaded(); },
+                                       has_cache, cache_vals, slab, slab_req, false, s, ar, hc);
         raise_verdict(u, r.bad, r.delta, r.full, has_cache, cache_vals);
         g_apply_hint.put(hint_key, ar.total);
         // the verdict is final, and the writes behind it are done (the downloads above followed them)
