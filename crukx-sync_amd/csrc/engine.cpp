@@ -1463,12 +1463,13 @@ PartCheck apply_part(const Update &u, const Layout &L, const ApplyPart &P, const
     unsigned int *n_more = ub.at<unsigned int>(i_nmore);
     uint8_t *multi = ar.get<uint8_t>(tiles);
     uint32_t *done = ar.get<uint32_t>(tiles);
-    // the verdict's inputs, set up before the select pass writes anything: between its writes and the
-    // commit that can undo them, the host only launches
+    // the verdict's inputs and the pinned memory of its result, set up before the select pass writes
+    // anything: between its writes and the commit that can undo them, the host only launches
     // (allocated in a dry pass too: a part's write pass then asks for exactly the buffers its dry pass had)
     uint64_t *d_want = ub.at<uint64_t>(i_want), *d_cached = ub.at<uint64_t>(i_cached);
     int32_t *d_has = ub.at<int32_t>(i_has);
     unsigned int *ok = ar.get<unsigned int>(1);
+    auto *result = reinterpret_cast<unsigned long long *>(t_stage.get((1 + 2 * (uint64_t)T) * sizeof(unsigned long long)));
     SelectArgs sa{d_descs, sd.tile_tensor, T, slab, hall, lb, d_gof, d_groups, local, rec, rstart, tchg, bad, more,
                   n_more, (uint32_t)std::min<uint64_t>(1024, (uint64_t)kSelMoreWindows * tiles), dz, sdelta, multi,
                   done, (uint32_t)C, blk_prefix, full};
@@ -1486,7 +1487,6 @@ PartCheck apply_part(const Update &u, const Layout &L, const ApplyPart &P, const
     launch_tensor_sums(d_descs, T, sdelta, full, tdelta, t_full, s);  // the select pass summed the cold slabs
     // the verdict on the device too, and the commit behind it (the remaining writes if the update
     // verifies, the undoing of the select pass's if not); the host waits for the verdict's data only
-    auto *result = reinterpret_cast<unsigned long long *>(t_stage.get((1 + 2 * (uint64_t)T) * sizeof(unsigned long long)));
     launch_verdict(T, reinterpret_cast<const unsigned long long *>(tdelta), t_full, d_has, d_cached, d_want, bad, ok,
                    result, s);
     if (!dry) {

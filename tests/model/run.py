@@ -307,8 +307,65 @@ def scenario_parts() -> None:
         print(f"parts {name}: {len(ref)} bytes as the oracle's; chained applies exact", flush=True)
 
 
+def scenario_pinned_exhausted() -> None:
+    """A call that runs out of pinned memory writes nothing: an update of many small tensors that does not
+    verify, applied by a thread whose pinned memory cannot grow past its first block, at the number of
+    tensors from which the call no longer fits there (found by bisection: up to it the verdict is
+    reported, from it on the failed allocation is)."""
+    import threading
+
+    import torch
+
+    import crukx_sync
+    import oracle
+    from crukx_sync import CorruptUpdate, _native
+
+    left = ctypes.c_int.in_dll(_native.lib(), "simt_host_mallocs_left")
+
+    def attempt(n: int) -> str:
+        """The error of an update of n tensors against a receiver whose last tensor is another; the
+        receiver is unchanged."""
+        old = {f"{i}": torch.full((8,), 0x3F80, dtype=torch.int16) for i in range(n)}
+        new = {k: v.clone() for k, v in old.items()}
+        for v in new.values():
+            v[3] += 1
+        upd = oracle.encode_update(old, new)
+        recv = {k: v.clone() for k, v in old.items()}
+        recv[f"{n - 1}"][5] ^= 1
+        want = {k: v.clone() for k, v in recv.items()}
+        got = []
+
+        def work():  # a thread of its own: its pinned memory starts empty
+            left.value = 1
+            try:
+                crukx_sync.apply_update(recv, upd)
+            except Exception as e:
+                got.append(e)
+            left.value = -1
+
+        t = threading.Thread(target=work)
+        t.start()
+        t.join()
+        assert all(torch.equal(recv[k], want[k]) for k in recv), f"{n} tensors, {got}: written"
+        if isinstance(got[0], CorruptUpdate):
+            return "verdict"
+        assert "hipHostMalloc" in str(got[0]), got
+        return "memory"
+
+    fits, fails = 3000, 4096
+    assert attempt(fits) == "verdict" and attempt(fails) == "memory"
+    while fails - fits > 1:
+        n = (fits + fails) // 2
+        if attempt(n) == "verdict":
+            fits = n
+        else:
+            fails = n
+        print(f"pinned memory: {n} tensors {'fit' if fits == n else 'do not fit'}", flush=True)
+    print(f"pinned memory: out of it from {fails} tensors on, nothing written", flush=True)
+
+
 SCENARIOS = {"parity": scenario_parity, "small4_flips": scenario_small4_flips, "rejected_early": scenario_rejected_early,
-             "group_message": scenario_group_message, "parts": scenario_parts,
+             "group_message": scenario_group_message, "parts": scenario_parts, "pinned_exhausted": scenario_pinned_exhausted,
              "device_offsets": scenario_device_offsets}
 
 if __name__ == "__main__":

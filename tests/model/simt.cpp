@@ -382,7 +382,12 @@ hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
 }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+// How many more pinned allocations succeed (negative: all), for tests of calls that run out of them.
+extern "C" int simt_host_mallocs_left;
+int simt_host_mallocs_left = -1;
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) {
+    if (simt_host_mallocs_left == 0) return hipErrorOutOfMemory;
+    if (simt_host_mallocs_left > 0) --simt_host_mallocs_left;
     return posix_memalign(p, 64, bytes ? bytes : 1) == 0 ? hipSuccess : hipErrorOutOfMemory;
 }
 hipError_t hipHostFree(void *p) {

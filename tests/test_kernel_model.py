@@ -76,3 +76,10 @@ def test_part_wise_encode_and_apply_match_the_oracle(model):
     rejected by the verification of the whole update with every tensor unchanged."""
     out = _run(model, "parts")
     assert out.count("chained applies exact") == 2 and out.count("rejected by the device passes") == 2
+
+
+def test_apply_that_runs_out_of_pinned_memory_writes_nothing(model):
+    """The last allocation of an apply comes before its first write: a call whose pinned memory cannot
+    grow fails with the receiver unchanged, whichever of its allocations is the one that fails."""
+    out = _run(model, "pinned_exhausted")
+    assert "nothing written" in out
