@@ -1357,6 +1357,12 @@ struct ApplyPart {
     uint64_t C = 0, B = 0, b0 = 0;
 };
 
+// Whether a part's blocks take a wavefront each or a lane each (a part's own bits are not looked up: the
+// whole payload's bound them).
+bool wave_decodes(const Update &u, const ApplyPart &P) {
+    return P.B <= kDecWaveBlocks && u.payload_len <= kDecWaveBits / 8;
+}
+
 // What one part's pass found: error flags, and per tensor of the part the checksum delta and (for
 // tensors without a cached checksum) the full checksum of the receiver's weights before the update.
 struct PartCheck {
@@ -1416,7 +1422,8 @@ PartCheck apply_part(const Update &u, const Layout &L, const ApplyPart &P, const
     hc.mark("apply_upload");
     Fork fork(s, tiles > kForkTiles);
     DecodeArgs da{d_descs, sh.pay, sh.pay_words, sh.bb + P.b0, sh.boff + P.b0, B, d_groups, (uint32_t)G, bmap,
-                  sh.lim, sh.off, sh.syms, sh.n_syms, dz, blk_sum, bad, sh.n_tables, sh.bit0, sh.lens};
+                  sh.lim, sh.off, sh.syms, sh.n_syms, dz, blk_sum, bad, sh.n_tables, sh.bit0,
+                  wave_decodes(u, P) ? sh.lens : nullptr};
     launch_decode(da, fork.aux);
     launch_scan_u64(blk_sum, B, blk_prefix, ar.get<unsigned long long>(scan_parts(B)), fork.aux);
 
@@ -1617,7 +1624,7 @@ void apply(const Update &u, const uint8_t *payload_dev, uint16_t *const *targets
     // code lengths by a code's first bits, for the decoder that small updates (or parts) take
     std::vector<uint8_t> lens;
     for (const ApplyPart &P : parts)
-        if (P.B <= kDecWaveBlocks && lens.empty()) lens.assign(u.tables.size() * kPeekLens, 0);
+        if (wave_decodes(u, P) && lens.empty()) lens.assign(u.tables.size() * kPeekLens, 0);
     for (size_t ti = 0; ti < lens.size() / kPeekLens; ++ti) {
         uint32_t from = 0;  // the codes of up to kPeekBits bits end at multiples of one peek
         for (uint32_t l = 1; l <= kPeekBits; ++l) {

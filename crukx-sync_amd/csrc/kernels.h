@@ -153,8 +153,8 @@ struct DecodeArgs {
     unsigned int *bad;
     uint32_t n_tables;              // tables: lim and off hold 17 entries each
     uint32_t bit0;                  // first payload bit in payload[0] (0-56, a multiple of 8)
-    // [tables][kPeekLens], for updates of at most kDecWaveBlocks blocks: the length of the code whose first
-    // kPeekBits bits are the index, or 0 when it is longer (or there is none)
+    // [tables][kPeekLens]: the length of the code whose first kPeekBits bits are the index, or 0 when it is
+    // longer (or there is none), for the decoder that takes a wavefront per block; null: a lane per block
     const uint8_t *lens;
 };
 
@@ -280,7 +280,9 @@ void launch_verdict(uint32_t n, const unsigned long long *delta, const uint64_t 
 void launch_tensor_sums(const TensorDesc *descs, uint32_t n_tensors, const uint64_t *a, const uint64_t *b,
                         uint64_t *out_a, uint64_t *out_b, hipStream_t s);
 void launch_decode(const DecodeArgs &a, hipStream_t s);
-constexpr uint64_t kDecWaveBlocks = 12288;  // updates of up to so many blocks: a wavefront per block
+constexpr uint32_t kSegBits = 3072;  // bits that a wavefront decodes at a time (RL-like blocks take about 2500)
+// updates of up to so many blocks, in a payload of up to so many bits: a wavefront per block
+constexpr uint64_t kDecWaveBlocks = 12288, kDecWaveBits = kDecWaveBlocks * kSegBits;
 constexpr uint32_t kDecSyms = 2048;  // decoding symbols staged in LDS when they fit (with the first indices)
 // Dynamic LDS of the decoder for n_syms symbols.
 inline uint32_t decode_lds_bytes(uint32_t n_syms, uint32_t n_tables) { return n_syms <= kDecSyms ? (n_syms + 17u * n_tables) * 4u : 0u; }

@@ -1479,15 +1479,21 @@ __device__ void decode_blocks(const DecodeArgs &a, const uint32_t *S_syms) {
 // LDS).  Composing that map with itself three times gives the position eight codes on, so the starts of
 // every eighth code follow in a chain of 32 LDS reads, the ones between from seven more, one lane per
 // chain.  With every start known, each lane decodes four consecutive changes and a wave scan of their
-// gaps gives the block-relative indices.  Codes that do not fit a 64-bit window (long unary runs) are
-// read from HBM one at a time when a chain reaches them.  It decodes some 2500 bit positions to find 256
+// gaps gives the block-relative indices.  A run of 32 ones or more ends where the run 32 bits on does, so
+// those positions take the next position of the one 32 bits on; a code whose run passes the segment begins
+// the next one, and codes of which a segment would hold fewer than eight are read from HBM by themselves,
+// the run by all lanes.  So the work follows the payload's bits, and updates of more than kSegBits bits per
+// block on average (kDecWaveBits) are left to the lanes as well.  It decodes some 2500 bit positions to find 256
 // codes, which only pays while the chip has room.  Measured (400 / 2,000 / 3,900 / 7,800 / 15,600 / 31,000
 // blocks, beside nothing else): 23 / 25 / 44 / 72 / 124 / 233 us, the lane-per-block decoder 142 / 141 / 141 /
 // 142 / 145 / 162; beside the cold histogram pass the two meet at about 12,000 blocks, where the line is.
-constexpr uint32_t kSegBits = 3072;      // bit positions per segment (RL-like blocks take about 2500 bits)
+// Updates of long codes (2048 of 66 / 202 / 1002 bits each, in 316 / 968 / 4,808 blocks), the whole apply:
+// 0.34 / 0.66 / 0.57 ms, the lane-per-block decoder 1.31 / 1.51 / 2.40 (with a segment begun after every run
+// of 32 or more 2.49 / 2.80 / 3.73).
 constexpr uint32_t kSegWords = kSegBits / 32 + 5;
-constexpr uint16_t kLongCode = 0xFFFF;   // next position of a code that does not fit its window (or is none)
-static_assert(kSegBits % 512 == 0 && kSegBits + 64 < kLongCode, "kSegBits");
+constexpr uint16_t kLongCode = 0xFFFF;   // next position of a code whose run passes the segment (or that is none)
+constexpr uint16_t kRunCode = 0xFFFE;    // ... of one whose run fills its first 32 bits, until it is known
+static_assert(kSegBits % 512 == 0 && kSegBits + 128 < kRunCode && kSegBits <= 64 * 64, "kSegBits");
 
 struct alignas(16) WaveDecodeLds {
     uint32_t w[kSegWords];      // the segment's payload from the word before its first bit's on, big-endian
@@ -1509,14 +1515,17 @@ __device__ __forceinline__ uint64_t stream_bits(const DecodeArgs &a, uint64_t po
     return s ? (h << s) | (l >> (64 - s)) : h;
 }
 
-// length of the unary run at pos: exact while it is at most qmax and ends before bit `end`, else larger
-// than qmax or reaching `end`
+// length of the unary run at pos, by the whole wavefront (64 words at a time): exact while it is at most
+// qmax and ends before bit `end`, else larger than qmax or reaching `end`
 __device__ uint64_t unary_run(const DecodeArgs &a, uint64_t pos, uint64_t end, uint64_t qmax) {
     uint64_t q = 0;
     for (;;) {
-        const uint64_t y = ~stream_bits(a, pos + q);
-        if (y) return q + (uint64_t)__builtin_clzll(y);
-        q += 64;
+        const uint64_t y = ~stream_bits(a, pos + q + 64 * lane()), m = ballot(y != 0);
+        if (m) {
+            const uint32_t l = (uint32_t)__builtin_ctzll(m), c = y ? (uint32_t)__builtin_clzll(y) : 0u;
+            return q + 64 * l + __builtin_amdgcn_readlane(c, l);
+        }
+        q += 64 * 64;
         if (q > qmax || pos + q >= end) return q;
     }
 }
@@ -1558,6 +1567,7 @@ __global__ __launch_bounds__(64) void k_decode_wave(DecodeArgs a) {
     uint64_t rel = 0;   // bits of the block before the next code
     bool bad = false;   // uniform
     bool off = false;   // this lane decoded a gap past the tensor
+    bool far = false;   // the last segment held fewer than eight codes (uniform)
     while (done < cnt && !bad) {  // a segment: at least one code each
         if (rel >= nbits) {
             bad = true;
@@ -1565,15 +1575,39 @@ __global__ __launch_bounds__(64) void k_decode_wave(DecodeArgs a) {
         }
         // positions [0, n) of the segment are decoded (whole rounds of 512), from bit `at` of the stream
         const uint64_t at = first + rel, w0 = at >> 5;
+        // the code at the segment's begin by itself, its run being q
+        auto read_one = [&](uint64_t q) {
+            uint64_t gap = 0;
+            uint32_t zz = 0;
+            bad = q > qmax || at + q >= end;
+            if (bad) return;
+            const uint32_t len = finish(q, stream_bits(a, at + q + 1), gap, zz);
+            bad = len > rice + 17 || gap >= size;
+            if (ln == 0) {
+                S.code[done] = (uint32_t)gap;
+                S.zz[done] = zz;
+            }
+            ++done;
+            rel += q + 1 + len;
+        };
+        if (far) {
+            const uint64_t q = unary_run(a, at, end, qmax);
+            far = q >= kSegBits / 8;
+            if (far) {
+                read_one(q);
+                continue;
+            }
+        }
         const uint32_t shift = (uint32_t)(at & 31), n = (uint32_t)min64(kSegBits, (nbits - rel + 511) & ~511ULL);
         const uint32_t *const p32 = reinterpret_cast<const uint32_t *>(a.payload);
         const uint64_t n32 = 2 * a.n_words;
         for (uint32_t i = ln; i < n / 32 + 4; i += 64) S.w[i + 1] = __builtin_bswap32(p32[min64(w0 + i, n32 - 1)]);
         wave_fence();
         // position 64 i + ln starts at the same bit s of its word for every i.  Its 64-bit window is two
-        // 32-bit funnel shifts by 32 - s, of the words from the one before it on where s is 0; a unary run
-        // that fills the first 32 bits is left to the chains.
+        // 32-bit funnel shifts by 32 - s, of the words from the one before it on where s is 0; what does
+        // not lie in it is read below.
         const uint32_t s = (shift + ln) & 31, wl = (shift + ln + 31) >> 5, rs = 32 - s;
+        uint64_t runs = 0;  // rows of 64 positions with runs of 32 or more
         for (uint32_t i0 = 0; i0 < n / 64; i0 += 4) {
             uint32_t len[4], peek[4], fixed[4];
             bool any = false;
@@ -1585,20 +1619,38 @@ __global__ __launch_bounds__(64) void k_decode_wave(DecodeArgs a) {
                 fixed[u] = q + 1 + rice;
                 peek[u] = (uint32_t)(((((uint64_t)hi << 32) | lo) << min(fixed[u], 63u)) >> 47);
                 len[u] = S.len[peek[u] >> (17 - kPeekBits)];
-                if (q == 32 || fixed[u] > 47) len[u] = 18;
+                if (q == 32 || fixed[u] > 47) len[u] = 0;
                 any = any || len[u] == 0;
             }
             if (ballot(any)) {
 #pragma unroll
-                for (uint32_t u = 0; u < 4; ++u) len[u] = len[u] ? len[u] : length_of(peek[u]);
+                for (uint32_t u = 0; u < 4; ++u) {
+                    const bool run = fixed[u] == 33 + rice;
+                    if (fixed[u] > 47) {  // the Huffman code lies past the window's first half: one word on
+                        const uint32_t *const w = &S.w[wl + 2 * (i0 + u)];
+                        const uint32_t lo = funnel_right(w[1], w[2], rs), lo2 = funnel_right(w[2], w[3], rs);
+                        peek[u] = (uint32_t)(((((uint64_t)lo << 32) | lo2) << (fixed[u] - 32)) >> 47);
+                    }
+                    len[u] = run ? 19u : len[u] ? len[u] : length_of(peek[u]);
+                    if (ballot(run)) runs |= 1ULL << (i0 + u);
+                }
             }
 #pragma unroll
             for (uint32_t u = 0; u < 4; ++u) {
                 const uint32_t p = 64 * (i0 + u) + ln;
-                S.next[p] = (uint16_t)(len[u] <= 17 ? p + fixed[u] + len[u] : (uint32_t)kLongCode);
+                S.next[p] = (uint16_t)(len[u] <= 17 ? p + fixed[u] + len[u] : len[u] == 18 ? (uint32_t)kLongCode : (uint32_t)kRunCode);
             }
         }
         wave_fence();
+        while (runs) {  // from the last such row back: the position 32 bits on is known
+            const uint32_t i = 63 - (uint32_t)__builtin_clzll(runs), p = 64 * i + ln;
+            runs &= ~(1ULL << i);
+#pragma unroll
+            for (uint32_t half = 2; half-- > 0;) {
+                if ((ln >> 5) == half && S.next[p] == kRunCode) S.next[p] = p + 32 < n ? S.next[p + 32] : kLongCode;
+                wave_fence();
+            }
+        }
         // jump = next composed with itself three times.  A code begins after the one before it, so an
         // in-place round in ascending order reads only entries that it has not written yet.
         for (int round = 0; round < 3; ++round) {
@@ -1632,64 +1684,73 @@ __global__ __launch_bounds__(64) void k_decode_wave(DecodeArgs a) {
                 c = S.next[c];
             }
         }
-        // then one at a time: the last codes of the block or segment, and a long one
+        // then one at a time: the last codes of the block or segment
         uint32_t found = done + 8 * chains;
-        bool is_long = false;
         while (found < cnt && pos < n) {
             const uint32_t to = __builtin_amdgcn_readfirstlane(S.next[pos]);
-            is_long = to == kLongCode;
-            if (is_long) break;
+            if (to == kLongCode) break;
             if (ln == 0) S.code[found] = pos;
             ++found;
             pos = to;
         }
         wave_fence();
-        // the codes found (the last one again past them), from the payload in LDS; all loads together
-        if (found > done) {
-            uint32_t zz[4];
-            uint64_t gap[4];
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) {
-                const uint32_t p = shift + S.code[min(done + 64 * u + ln, found - 1)], *const w = &S.w[(p >> 5) + 1], sh = p & 31;
-                const uint64_t hl = ((uint64_t)w[0] << 32) | w[1], x = sh ? (hl << sh) | (w[2] >> (32 - sh)) : hl;
-                const uint32_t q = (uint32_t)__builtin_clzll(~x);
-                finish(q, x << (q + 1), gap[u], zz[u]);
-                off = off || q > qmax || gap[u] >= size;
-            }
+        far = found < done + 8;
+        if (!pos) {  // the first code passes the segment
+            read_one(unary_run(a, at, end, qmax));
             wave_fence();
+            continue;
+        }
+        // the codes found (the last one again past them), from the payload in LDS; all loads together
+        auto window = [&](uint32_t p) {  // the 64 bits from bit p of S.w[1] on
+            const uint32_t *const w = &S.w[(p >> 5) + 1], sh = p & 31;
+            const uint64_t hl = ((uint64_t)w[0] << 32) | w[1];
+            return sh ? (hl << sh) | (w[2] >> (32 - sh)) : hl;
+        };
+        uint32_t zz[4], q[4];
+        uint64_t gap[4], x[4];
+        bool any = false;
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            x[u] = window(shift + S.code[min(done + 64 * u + ln, found - 1)]);
+            q[u] = ~x[u] ? (uint32_t)__builtin_clzll(~x[u]) : 64u;
+            any = any || q[u] + 1 + rice > 47;
+        }
+        if (ballot(any)) {  // remainder and code not both in the window: the run's end, then a window of their own
 #pragma unroll
             for (uint32_t u = 0; u < 4; ++u) {
-                const uint32_t i = done + 64 * u + ln;
-                if (i < found) {
-                    S.code[i] = (uint32_t)gap[u];
-                    S.zz[i] = zz[u];
+                const uint32_t p = shift + S.code[min(done + 64 * u + ln, found - 1)];
+                while (q[u] % 64 == 0 && q[u]) {  // every run in the map ends in the segment's words
+                    const uint64_t y = ~window(p + q[u]);
+                    q[u] += y ? (uint32_t)__builtin_clzll(y) : 64u;
+                    if (y) break;
                 }
+                x[u] = window(p + q[u] + 1);
+            }
+        } else {
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) x[u] <<= q[u] + 1;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            finish(q[u], x[u], gap[u], zz[u]);
+            off = off || q[u] > qmax || gap[u] >= size;
+        }
+        wave_fence();
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            const uint32_t i = done + 64 * u + ln;
+            if (i < found) {
+                S.code[i] = (uint32_t)gap[u];
+                S.zz[i] = zz[u];
             }
         }
         done = found;
-        if (is_long) {  // the next segment begins after it
-            const uint64_t cur = at + pos, q = unary_run(a, cur, end, qmax);
-            uint64_t gap = 0;
-            uint32_t zz = 0;
-            bad = q > qmax || cur + q >= end;
-            if (!bad) {
-                const uint32_t len = finish(q, stream_bits(a, cur + q + 1), gap, zz);
-                bad = len > rice + 17 || gap >= size;
-                if (ln == 0) {
-                    S.code[done] = (uint32_t)gap;
-                    S.zz[done] = zz;
-                }
-                ++done;
-                rel += pos + q + 1 + len;
-                pos = 0;
-            }
-        }
         rel += pos;
         wave_fence();
     }
     // the codes' lengths add up to the block's: each ends inside it
-    const bool far = ballot(off) != 0;
-    bad = bad || rel != nbits || far;
+    const bool past = ballot(off) != 0;
+    bad = bad || rel != nbits || past;
     unsigned long long sum = 0;
     if (!bad) {
         // changes 4 ln .. 4 ln + 3: their gaps summed along the block
@@ -2679,7 +2740,7 @@ void launch_tensor_sums(const TensorDesc *descs, uint32_t n_tensors, const uint6
 }
 
 void launch_decode(const DecodeArgs &a, hipStream_t s) {
-    if (a.n_blocks <= kDecWaveBlocks) {
+    if (a.lens) {
         CRX_LAUNCH("decode", k_decode_wave, (uint32_t)a.n_blocks, 64, s, a);
         return;
     }

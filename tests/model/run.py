@@ -364,8 +364,72 @@ def scenario_pinned_exhausted() -> None:
     print(f"pinned memory: out of it from {fails} tensors on, nothing written", flush=True)
 
 
+def launches() -> list:
+    """The kernel launches since the last call: (workgroups, work-items each, collectives) of each."""
+    from crukx_sync import _native
+    f = _native.lib().simt_launches
+    f.restype, f.argtypes = ctypes.c_uint64, [ctypes.c_void_p, ctypes.c_uint64]
+    buf = (ctypes.c_uint64 * 30000)()
+    return [tuple(buf[3 * i:3 * i + 3]) for i in range(f(buf, 10000))]
+
+
+def scenario_long_codes() -> None:
+    """Blocks of unary runs past a 64-bit window (a dense run and changes `spread` apart in one exponent
+    group, whose Rice parameter suits neither): exact, rejected when a payload byte is flipped, and the
+    wave decoder's work grows with the payload's bits and not with the number of such codes."""
+    import torch
+
+    import crukx_sync
+    import oracle
+    import scenarios
+    from crukx_sync import _native, codec
+
+    per_bit = {}
+    for spread, far in ((8, 2048), (40, 2048), (64, 2048), (200, 1024), (2000, 256), (4000, 128)):
+        dense = int(0.6 * far * spread)
+        n = far * spread + dense
+        a = torch.full((n,), 0x3F80, dtype=torch.int16)
+        b = a.clone()
+        b[:dense] += 1
+        b[dense::spread] += 3
+        upd = oracle.encode_update({"w": a}, {"w": b})
+        u = crukx_sync.parse(upd)
+        blocks = _native.lib().crx_update_n_blocks(u.handle)
+        pay = _native.lib().crx_update_payload_len(u.handle)
+        chk = {"w": (codec.checksum(a), a._version)}
+        launches()
+        w = {"w": a}
+        crukx_sync.apply_update(w, upd, chk)
+        assert torch.equal(a, b)
+        decode = [c for g, t, c in launches() if g == blocks and t == 64]
+        assert len(decode) >= 1
+        per_bit[spread] = max(decode) / (8 * pay + 512 * blocks)
+        print(f"long codes {spread}: {blocks} blocks, {8 * pay // blocks} bits each: {max(decode)} collectives, "
+              f"{per_bit[spread]:.3f} per bit", flush=True)
+        if spread in (64, 4000):
+            w["w"].copy_(torch.full((n,), 0x3F80, dtype=torch.int16))
+            want = w["w"].clone()
+            for at in range(len(upd) - pay, len(upd), pay // 6):
+                bad = bytearray(upd)
+                bad[at] ^= 0x41
+                try:
+                    crukx_sync.apply_update(w, bytes(bad))
+                except crukx_sync.CorruptUpdate:
+                    pass
+                else:
+                    raise AssertionError(f"byte {at} flipped: applied")
+                assert torch.equal(w["w"], want)
+    a, b = scenarios.far_pair()
+    crukx_sync.apply_update({"w": a}, oracle.encode_update({"w": a}, {"w": b}))
+    assert torch.equal(a, b)
+    # a block is decoded in segments of whole 512-bit rounds (hence 512 bits more per block)
+    assert max(per_bit.values()) < 3 * per_bit[8], per_bit
+    print("long codes: work in proportion to the bits", flush=True)
+
+
 SCENARIOS = {"parity": scenario_parity, "small4_flips": scenario_small4_flips, "rejected_early": scenario_rejected_early,
-             "group_message": scenario_group_message, "parts": scenario_parts, "pinned_exhausted": scenario_pinned_exhausted,
+             "group_message": scenario_group_message, "parts": scenario_parts, "long_codes": scenario_long_codes,
+             "pinned_exhausted": scenario_pinned_exhausted,
              "device_offsets": scenario_device_offsets}
 
 if __name__ == "__main__":

@@ -76,6 +76,11 @@ struct Fiber {
     uint32_t arg = 0;
 };
 
+// A launch that ended: its workgroups, work-items per workgroup, and the collectives its wavefronts passed.
+struct Launch {
+    uint64_t grid, block, collectives;
+};
+
 constexpr size_t kStackBytes = 128 << 10;
 Fiber g_pool[1024];  // the work-items of the running workgroup
 uint32_t g_n = 0;
@@ -89,6 +94,7 @@ void *g_ctx = nullptr;
 uint8_t *g_dyn = nullptr;
 uint64_t g_launches = 0;
 uint64_t g_resolves = 0, g_switches = 0;
+std::vector<Launch> g_log;
 const int g_stack_fill = std::getenv("SIMT_STACK_FILL") ? (int)std::strtol(std::getenv("SIMT_STACK_FILL"), nullptr, 0) : -1;
 constexpr size_t kStackFill = 32 << 10;
 const int g_lds_fill = std::getenv("SIMT_LDS_FILL") ? (int)std::strtol(std::getenv("SIMT_LDS_FILL"), nullptr, 0) : 0xA5;
@@ -339,6 +345,7 @@ void run(dim3 grid, dim3 block, size_t dyn_bytes, void (*body)(void *), void *ct
         schedule();
     }
     g_dyn = nullptr;
+    if (g_log.size() < 100000) g_log.push_back(Launch{grid.x, block.x, g_resolves - r0});
     if (profile)
         std::fprintf(stderr, "simt: launch %llu body %p grid %u block %u: %llu collectives, %llu switches: %.1f ms\n",
                      (unsigned long long)g_launches, (void *)body, grid.x, block.x,
@@ -347,6 +354,14 @@ void run(dim3 grid, dim3 block, size_t dyn_bytes, void (*body)(void *), void *ct
 }
 
 }  // namespace simt
+
+// The launches since the last call, oldest first, at most `cap` of them: three numbers each (Launch).
+extern "C" uint64_t simt_launches(uint64_t *out, uint64_t cap) {
+    const uint64_t n = std::min<uint64_t>(cap, simt::g_log.size());
+    std::memcpy(out, simt::g_log.data(), n * sizeof(simt::Launch));
+    simt::g_log.clear();
+    return n;
+}
 
 // ------------------------------------------------------------------ host runtime
 struct simt_stream {

@@ -113,3 +113,16 @@ def chain_cache(steps=5):
         w = w + 1e-6 * torch.sign(torch.randn(w.shape, generator=g))
         states.append({"w": w.bfloat16()})
     return states
+
+
+def far_pair():
+    """Changes 40,000 apart with a few 31 to 64 times 2^16 apart: the group's Rice parameter is 16, and the far
+    codes' runs and remainders pass 47 bits, with runs below and above 32."""
+    gaps = [40_000 + 331 * (i % 7) for i in range(400)]
+    for i, k in enumerate((31 * 65536 + 5, 40 * 65536 + 77, 31 * 65536 + 60000, 33 * 65536, 32 * 65536 - 1, 64 * 65536)):
+        gaps.insert(60 * i + 7, k)
+    at = torch.tensor(gaps).cumsum(0)
+    a = torch.full((int(at[-1]) + 100,), 0x3F80, dtype=torch.int16)
+    b = a.clone()
+    b[at] += torch.arange(len(gaps), dtype=torch.int16) % 50 + 1
+    return a, b

@@ -97,6 +97,19 @@ def test_decoder_by_number_of_blocks(tensors, form):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,lanes", [(1_900_000, False), (2_900_000, True)])
+def test_decoder_by_bits_of_the_payload(n, lanes):
+    """Updates of few enough blocks for a wavefront each, in payloads on both sides of 12288 * 3072 bits."""
+    old, new = _many_groups(1, n)
+    upd = crukx_sync.encode_update(_cuda(old), _cuda(new))
+    u, L = crukx_sync.parse(upd), _native.lib()
+    assert L.crx_update_n_blocks(u.handle) <= 12288 and (8 * L.crx_update_payload_len(u.handle) > 12288 * 3072) == lanes
+    recv = _cuda(old)
+    crukx_sync.apply_update(recv, upd)
+    assert torch.equal(recv["t0"].cpu(), new["t0"])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("spread", [3, 700, 9_001, 120_000])
 def test_blocks_of_long_codes(spread):
     """Blocks of one to many decoder segments, with unary runs past a 64-bit window: changes in dense runs
@@ -110,6 +123,17 @@ def test_blocks_of_long_codes(spread):
     upd = crukx_sync.encode_update(_cuda(old), _cuda(new))
     assert upd == oracle.encode_update(old, new)
     recv = _cuda(old)
+    crukx_sync.apply_update(recv, upd)
+    assert torch.equal(recv["w"].cpu(), b)
+
+
+@pytest.mark.gpu
+def test_blocks_of_long_remainders():
+    a, b = scenarios.far_pair()
+    upd = crukx_sync.encode_update({"w": a.cuda()}, {"w": b.cuda()})
+    assert upd == oracle.encode_update({"w": a}, {"w": b})
+    assert crukx_sync.parse(upd).tensors[0].groups[0].rice_r == 16
+    recv = {"w": a.cuda()}
     crukx_sync.apply_update(recv, upd)
     assert torch.equal(recv["w"].cpu(), b)
 

@@ -83,3 +83,11 @@ def test_apply_that_runs_out_of_pinned_memory_writes_nothing(model):
     grow fails with the receiver unchanged, whichever of its allocations is the one that fails."""
     out = _run(model, "pinned_exhausted")
     assert "nothing written" in out
+
+
+def test_long_codes_cost_the_wave_decoder_their_bits(model):
+    """Updates whose blocks hold unary runs of 40 to 4000 bits: exact, rejected when corrupted, and the
+    decoder's work is in proportion to the payload's bits (it once built a segment's map again for each
+    such code: 0.38 collectives per bit instead of 0.06)."""
+    out = _run(model, "long_codes")
+    assert "work in proportion to the bits" in out
