@@ -28,6 +28,24 @@ def test_count_slab_follows_the_size():
     assert [f(1 << 32, s) for s in (1, 128, 1000, 4096, 1 << 14)] == [128, 128, 896, 4096, 1 << 14]
 
 
+@pytest.mark.parametrize("n,kept,want", [
+    (1_700_000, 512, 65536), (12_800_000, 4096, 65536), (26_600_000, 8192, 65536), (100_000_000, 32768, 32768)])
+def test_count_slab_of_a_whole_model_applied_in_pieces_before(n, kept, want):
+    """A model of 7.6 billion weights after applies of its tensors (n weights) one by one: its slabs are the
+    whole's again (or half of them, whose counts are used), and a piece's thereafter too."""
+    L, pieces = _native.lib(), 7_600_000_000 // n
+    changes = 76_000_000
+    assert L.crx_apply_count_slab(n, n // 100, 1 << 24) == kept
+    assert codec._count_slab(changes, [kept] * pieces, [n] * pieces, 1 << 24) == want
+    assert codec._count_slab(changes, [kept, 65536] * (pieces // 2), [n] * (pieces // 2 * 2), 1 << 24) == (want if 2 * kept >= want else 65536)
+    assert codec._count_slab(changes, [], [n] * pieces, 1 << 24) == 65536
+    assert codec._count_slab(n // 100, [want], [n], 1 << 24) == want
+    assert codec._count_slab(n // 100, [kept], [n], 1 << 24) == kept
+    # the same tensors at a few more changes or elements than the rule's lines: their counts are used
+    assert codec._count_slab(changes * 3, [65536] * pieces, [n] * pieces, 1 << 24) == 65536
+    assert codec._count_slab(changes, [32768] * pieces, [n] * pieces, 1 << 24) == 32768
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 511, 512, 513, 512 * 128, 512 * 128 + 1, 512 * 2048, 512 * 2048 + 1, 512 * 4096,
                                512 * 4096 + 1])
