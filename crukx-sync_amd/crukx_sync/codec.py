@@ -350,10 +350,19 @@ _COUNT_CACHE = True
 
 # Receiver-side exponent counts per slab, kept on the device across updates of the same tensors:
 # id(tensor) -> (weakref, _version after our last write, device buffer, _SLAB, device, buffer address,
-# slab size of the counts).  They are used only with the same _SLAB, in an apply that ranks slabs of that
+# slab size of the counts, bytes under the limit below).  They are used only with the same _SLAB, in an apply that ranks slabs of that
 # size, and with a checksum-cache hit for the tensor (the same trust rule), and let apply skip its full
 # read of those weights (crx_apply_counts).
 _hist = {}
+# Counts take 1 KiB per slab: at most 1/64 of the weights' bytes in the slabs of 32768 and 65536 elements
+# that calls of 2^26 weights and more take, but as much as the weights themselves in slabs of 512.  All
+# counts of smaller slabs together (smaller than the largest that _SLAB allows) take at most
+# _FINE_COUNTS bytes, which holds every call's while a receiver's calls are few and whole; a model streamed
+# through apply tensor by tensor keeps those of its first tensors and reads the others' weights at every
+# update (1.5B weights in 338 calls: 473 MB of counts without the limit, 74 MB with it, the 338 calls
+# 69-72 and 72 ms).
+_COARSE_SLAB, _FINE_COUNTS = 32768, 64 << 20
+_fine = 0  # bytes of those kept
 # Guards _hist across threads.  Reentrant: a weakref callback that drops an entry can run inside a
 # locked region when a garbage collection happens there.
 _hist_lock = threading.RLock()
@@ -367,9 +376,17 @@ def _hist_lookup(t):
     return e
 
 
+def _hist_drop(key):
+    """Forget the counts of id `key` (the caller holds _hist_lock)."""
+    global _fine
+    e = _hist.pop(key, None)
+    if e is not None:
+        _fine -= e[7]
+
+
 def _hist_forget(key):
     with _hist_lock:
-        _hist.pop(key, None)
+        _hist_drop(key)
 
 
 def _apply_inputs(names, numels, weights, checksums):
@@ -424,12 +441,17 @@ def _count_slab(changes, sizes, numels, slab):
     return suits
 
 
-def _hist_store(t, buf, slab, dev, size):
-    """Record counts for t (the caller holds _hist_lock)."""
-    key = id(t)
+def _hist_store(t, buf, slab, dev, size, fine):
+    """Record counts for t (the caller holds _hist_lock), unless they are fine ones (smaller slabs) that
+    other threads' applies have left no room for."""
+    global _fine
+    key, fine = id(t), 4 * buf.numel() if fine else 0
     e = _hist.get(key)
     ref = e[0] if e is not None and e[0]() is t else weakref.ref(t, lambda _r, key=key: _hist_forget(key))
-    _hist[key] = (ref, t._version, buf, slab, dev, buf.data_ptr(), size)
+    _hist_drop(key)
+    if not fine or _fine + fine <= _FINE_COUNTS:
+        _fine += fine
+        _hist[key] = (ref, t._version, buf, slab, dev, buf.data_ptr(), size, fine)
 
 
 def _cache_get(checksums, name, t):
@@ -516,7 +538,7 @@ def apply(weights: Mapping[str, torch.Tensor], u: Update, checksums: dict | None
             for a, c, v in zip(targets, has, vers):
                 e = hg(id(a)) if c else None
                 if e is not None:
-                    ref, ver, buf, sl, on, at, k = e
+                    ref, ver, buf, sl, on, at, k, _ = e
                     if ver == v and sl == slab and on == dev and ref() is a:
                         bufs.append(buf)
                         hist_in.append(at)
@@ -526,6 +548,7 @@ def apply(weights: Mapping[str, torch.Tensor], u: Update, checksums: dict | None
                 hist_in.append(0)
                 sizes.append(0)
     size = _count_slab(L.crx_update_total_changes(u.handle), sizes, numels, slab)
+    fine = False
     if keep:
         fresh = []  # tensors without counts of this slab size
         if sizes.count(size) != len(sizes):
@@ -535,6 +558,18 @@ def apply(weights: Mapping[str, torch.Tensor], u: Update, checksums: dict | None
         hist_out = list(hist_in)
         # tensors without usable counts: one allocation, sliced per tensor
         fresh = [(i, L.crx_apply_hist_words(targets[i].numel(), size)) for i in fresh]
+        if fresh:
+            fine = size < min(_COARSE_SLAB, L.crx_apply_count_slab(1 << 40, 0, slab))
+            with _hist_lock:
+                for i, _ in fresh:
+                    _hist_drop(id(targets[i]))
+                room = _FINE_COUNTS - _fine if fine else None
+            if fine:
+                wanted, fresh = fresh, []
+                for i, w in wanted:
+                    if 4 * w <= room:
+                        room -= 4 * w
+                        fresh.append((i, w))
         if fresh:
             block = torch.empty(sum(w for _, w in fresh), dtype=torch.int32, device=dev)
             at, base = 0, block.data_ptr()
@@ -555,7 +590,7 @@ def apply(weights: Mapping[str, torch.Tensor], u: Update, checksums: dict | None
     if rc != _native.OK:
         with _hist_lock:
             for a in targets:  # their counts may be half-updated
-                _hist.pop(id(a), None)
+                _hist_drop(id(a))
         if rc == _native.DEVICE and staged is targets:
             # a runtime error may come after the verified writes were enqueued: the weights may have
             # changed, so cached checksums of them must no longer be trusted (a new _version does that)
@@ -573,10 +608,12 @@ def apply(weights: Mapping[str, torch.Tensor], u: Update, checksums: dict | None
             hg = _hist.get
             for a, buf, v in zip(targets, bufs, after):
                 e = hg(id(a))
+                if buf is None:
+                    continue
                 if e is not None and e[2] is buf and e[0]() is a:  # the same counts: a new version only
-                    _hist[id(a)] = (e[0], v, buf, slab, dev, e[5], size)
+                    _hist[id(a)] = (e[0], v, buf, slab, dev, e[5], size, e[7])
                 else:
-                    _hist_store(a, buf, slab, dev, size)
+                    _hist_store(a, buf, slab, dev, size, fine)
     if checksums is not None:  # record the version after our own write
         checksums.update({name: (c, v) for name, c, v in zip(names, header_chk, after)})
     return changed.value

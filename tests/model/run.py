@@ -427,8 +427,72 @@ def scenario_long_codes() -> None:
     print("long codes: work in proportion to the bits", flush=True)
 
 
+def scenario_kept_counts() -> None:
+    """The counts that a receiver keeps stay within their limit however many of its tensors are applied in
+    calls of their own, are used where they are kept, and give their room back with their tensors; every
+    apply is exact, of each tensor alone and of all together."""
+    import torch
+
+    import crukx_sync
+    import oracle
+    import scenarios
+    from crukx_sync import codec
+
+    codec._FINE_COUNTS = 24 << 10
+    states = [{}, {}]
+    for i in range(12):
+        states[0][f"t{i}"], states[1][f"t{i}"] = scenarios.rl_pair(3000, lr=4e-5, seed=70 + i)  # 6 slabs: 6 KiB
+
+    def kept():
+        return sum(4 * e[2].numel() for e in codec._hist.values())
+
+    def exact(names, s):
+        for k in names:
+            assert torch.equal(recv[k].view(torch.int16), states[s][k].view(torch.int16)), k
+
+    recv, chk = {k: v.clone() for k, v in states[0].items()}, {}
+    for s in (1, 0, 1):
+        for k in recv:
+            a, b = {k: states[1 - s][k]}, {k: states[s][k]}
+            crukx_sync.apply_update(recv, oracle.encode_update(a, b), chk)
+            assert kept() == codec._fine <= codec._FINE_COUNTS, (k, kept())
+        exact(recv, s)
+    assert sorted(codec._hist) == sorted(id(recv[f"t{i}"]) for i in range(4))
+    bufs = {k: e[2] for k, e in codec._hist.items()}
+    for s in (0, 1):
+        crukx_sync.apply_update(recv, oracle.encode_update(states[1 - s], states[s]), chk)
+        exact(recv, s)
+        assert kept() == codec._fine <= codec._FINE_COUNTS
+    assert all(codec._hist[k][2] is b for k, b in bufs.items())
+    del bufs
+    for k in ("t0", "t2"):
+        del recv[k], states[0][k], states[1][k]
+    assert kept() == codec._fine == 12 << 10
+    bad = bytearray(oracle.encode_update(states[1], states[0]))
+    bad[-9] ^= 0x20
+    try:
+        crukx_sync.apply_update(recv, bytes(bad), chk)
+    except crukx_sync.CorruptUpdate:
+        assert kept() == codec._fine == 0
+    else:
+        raise AssertionError("a corrupted update applied")
+    for s in (0, 1):
+        crukx_sync.apply_update(recv, oracle.encode_update(states[1 - s], states[s]), chk)
+        exact(recv, s)
+        assert kept() == codec._fine == 24 << 10
+    # slabs as large as _SLAB allows are not under the limit
+    codec._SLAB = 512
+    for s in (0, 1):
+        crukx_sync.apply_update(recv, oracle.encode_update(states[1 - s], states[s]), chk)
+        exact(recv, s)
+        assert kept() == 60 << 10 and codec._fine == 0
+    del recv
+    assert kept() == codec._fine == 0
+    print("kept counts: within the limit", flush=True)
+
+
 SCENARIOS = {"parity": scenario_parity, "small4_flips": scenario_small4_flips, "rejected_early": scenario_rejected_early,
-             "group_message": scenario_group_message, "parts": scenario_parts, "long_codes": scenario_long_codes,
+             "group_message": scenario_group_message, "parts": scenario_parts, "long_codes": scenario_long_codes, "kept_counts": scenario_kept_counts,
              "pinned_exhausted": scenario_pinned_exhausted,
              "device_offsets": scenario_device_offsets}
 

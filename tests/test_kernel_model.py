@@ -91,3 +91,9 @@ def test_long_codes_cost_the_wave_decoder_their_bits(model):
     such code: 0.38 collectives per bit instead of 0.06)."""
     out = _run(model, "long_codes")
     assert "work in proportion to the bits" in out
+
+
+def test_kept_counts_stay_within_their_limit(model):
+    """Tensors applied in calls of their own keep exponent counts of slabs as small as 512 elements, as
+    many bytes as their weights: all of a process's together are limited."""
+    assert "within the limit" in _run(model, "kept_counts")
