@@ -398,21 +398,24 @@ struct Arena {
     }
 };
 
-// Workspace bytes of the last call of one kind and its size key (e.g. its slab count): a following
-// call with a key within 1/16 of it reserves that much (plus 1/32) in one allocation, instead of one
-// trip through the caller's allocator per large buffer.  Only a hint: a call that needs more
-// allocates the rest buffer by buffer.
+// Workspace bytes of the last call of one kind with its slab size and size key (e.g. its slab count): a
+// following call of the same slab size with a key within 1/16 of it reserves that much (plus 1/32) in one
+// allocation, instead of one trip through the caller's allocator per large buffer.  (The slab count alone
+// says little: slabs grow with the call, and 2M weights have as many as 134M.)  Only a hint: a call that
+// needs more allocates the rest buffer by buffer.
 struct ArenaHint {
     std::mutex m;
+    uint32_t slab = 0;
     uint64_t key = 0, bytes = 0;
 
-    uint64_t get(uint64_t k) {
+    uint64_t get(uint32_t sl, uint64_t k) {
         std::lock_guard<std::mutex> g(m);
-        if (!key || k + k / 16 < key || key + key / 16 < k) return 0;
+        if (!key || sl != slab || k + k / 16 < key || key + key / 16 < k) return 0;
         return bytes + bytes / 32;
     }
-    void put(uint64_t k, uint64_t b) {
+    void put(uint32_t sl, uint64_t k, uint64_t b) {
         std::lock_guard<std::mutex> g(m);
+        slab = sl;
         key = k;
         bytes = b;
     }
@@ -1197,7 +1200,7 @@ void encode(int32_t n, const uint16_t *const *olds, const uint16_t *const *news,
     }
     const uint32_t T = (uint32_t)L.descs.size(), tiles = L.tiles;
     const uint64_t hint_key = tiles;
-    ar.reserve(g_encode_hint.get(hint_key));
+    ar.reserve(g_encode_hint.get(slab, hint_key));
     hc.mark("enc_layout");
 
     Ranked R = rank_changes(L, slab, s, ar, &hc, 1ULL << 32);
@@ -1321,7 +1324,7 @@ void encode(int32_t n, const uint16_t *const *olds, const uint16_t *const *news,
     const unsigned int hovf = (unsigned int)last[1];  // the flags' half of the word
     if (hovf & 2u || last[0] != total_bits) throw DeviceError("the packed payload's size differs from its codes' lengths");
     if (hovf) throw Invalid("a block exceeds 2^32 bits; the update cannot be represented");
-    g_encode_hint.put(hint_key, ar.total);
+    g_encode_hint.put(slab, hint_key, ar.total);
     E.d_block_bits = bb;
     E.payload_len = (total_bits + 7) / 8;
     E.d_payload = reinterpret_cast<const uint8_t *>(words);
@@ -1560,7 +1563,7 @@ void apply(const Update &u, const uint8_t *payload_dev, uint16_t *const *targets
         split ? split_parts(L, forced ? forced : kPartElements) : std::vector<std::pair<uint32_t, uint32_t>>{{0, T}};
     const uint32_t tiles = L.tiles;
     const uint64_t hint_key = (uint64_t)tiles + C / 256;
-    if (!split) ar.reserve(g_apply_hint.get(hint_key));
+    if (!split) ar.reserve(g_apply_hint.get(slab, hint_key));
     hc.mark("apply_layout");
 
     // groups, decoding tables and the group lookup (codec.py:594-625)
@@ -1709,7 +1712,7 @@ void apply(const Update &u, const uint8_t *payload_dev, uint16_t *const *targets
         const PartCheck r = apply_part(u, L, parts[0], sh, together ? tb : ub, [&] { if (together) uploaded(); },
                                        has_cache, cache_vals, slab, slab_req, false, s, ar, hc);
         raise_verdict(u, r.bad, r.delta, r.full, has_cache, cache_vals);
-        g_apply_hint.put(hint_key, ar.total);
+        g_apply_hint.put(slab, hint_key, ar.total);
         // the verdict is final, and the writes behind it are done (the downloads above followed them)
         *changed = C;
         return;

@@ -207,3 +207,30 @@ def test_packed_tensors_at_odd_elements(leads, cached):
         assert torch.equal(a[k].cpu().view(torch.int16), old[k].view(torch.int16))
         assert torch.equal(b[k].cpu().view(torch.int16), new[k].view(torch.int16))
         assert chk is None or chk[k] == oracle.checksum(new[k])
+
+
+@pytest.mark.gpu
+def test_a_small_calls_workspace_after_a_large_call_of_as_many_slabs():
+    """134 million weights in slabs of 32768 and 2 million in slabs of 512 are as many slabs: the small
+    encode and apply take no more memory after the large ones than after their like."""
+    def peaks(n):
+        a = torch.zeros(n, dtype=torch.int16, device="cuda")
+        b = a.clone()
+        b[::100] += 1
+        out = []
+        for f in (lambda: crukx_sync.encode_update_device({"w": a}, {"w": b}), lambda: crukx_sync.apply_update({"w": a}, upd)):
+            torch.cuda.synchronize()
+            torch.cuda.reset_peak_memory_stats()
+            before = torch.cuda.memory_allocated()
+            upd = f()
+            out.append(torch.cuda.max_memory_allocated() - before)
+        assert torch.equal(a, b)
+        return out
+
+    small, large = 2_090_000, 134_000_000
+    peaks(small)
+    alone = peaks(small)
+    peaks(large)
+    after = peaks(small)
+    # without a hint of its own size a call takes its workspace in chunks of 8 MiB, the last not full
+    assert all(x <= y + (8 << 20) for x, y in zip(after, alone)), (alone, after)
