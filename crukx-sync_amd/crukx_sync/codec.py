@@ -350,7 +350,7 @@ _COUNT_CACHE = True
 
 # Receiver-side exponent counts per slab, kept on the device across updates of the same tensors:
 # id(tensor) -> (weakref, _version after our last write, device buffer, _SLAB, device, buffer address,
-# slab size of the counts, bytes under the limit below).  They are used only with the same _SLAB, in an apply that ranks slabs of that
+# slab size of the counts).  They are used only with the same _SLAB, in an apply that ranks slabs of that
 # size, and with a checksum-cache hit for the tensor (the same trust rule), and let apply skip its full
 # read of those weights (crx_apply_counts).
 _hist = {}
@@ -376,12 +376,18 @@ def _hist_lookup(t):
     return e
 
 
+def _fine_slab(slab, size):
+    """Whether counts of slabs of `size` elements are under the limit, with _SLAB = slab (also called when a
+    tensor dies, as late as the interpreter's end: no library call)."""
+    return size < _COARSE_SLAB and not 0 < slab < size + 128
+
+
 def _hist_drop(key):
     """Forget the counts of id `key` (the caller holds _hist_lock)."""
     global _fine
     e = _hist.pop(key, None)
-    if e is not None:
-        _fine -= e[7]
+    if e is not None and _fine_slab(e[3], e[6]):
+        _fine -= 4 * e[2].numel()
 
 
 def _hist_forget(key):
@@ -441,17 +447,17 @@ def _count_slab(changes, sizes, numels, slab):
     return suits
 
 
-def _hist_store(t, buf, slab, dev, size, fine):
-    """Record counts for t (the caller holds _hist_lock), unless they are fine ones (smaller slabs) that
-    other threads' applies have left no room for."""
+def _hist_store(t, buf, slab, dev, size):
+    """Record counts for t (the caller holds _hist_lock), unless they are under the limit and other
+    threads' applies have left no room for them."""
     global _fine
-    key, fine = id(t), 4 * buf.numel() if fine else 0
+    key, fine = id(t), 4 * buf.numel() if _fine_slab(slab, size) else 0
     e = _hist.get(key)
     ref = e[0] if e is not None and e[0]() is t else weakref.ref(t, lambda _r, key=key: _hist_forget(key))
     _hist_drop(key)
     if not fine or _fine + fine <= _FINE_COUNTS:
         _fine += fine
-        _hist[key] = (ref, t._version, buf, slab, dev, buf.data_ptr(), size, fine)
+        _hist[key] = (ref, t._version, buf, slab, dev, buf.data_ptr(), size)
 
 
 def _cache_get(checksums, name, t):
@@ -538,7 +544,7 @@ def apply(weights: Mapping[str, torch.Tensor], u: Update, checksums: dict | None
             for a, c, v in zip(targets, has, vers):
                 e = hg(id(a)) if c else None
                 if e is not None:
-                    ref, ver, buf, sl, on, at, k, _ = e
+                    ref, ver, buf, sl, on, at, k = e
                     if ver == v and sl == slab and on == dev and ref() is a:
                         bufs.append(buf)
                         hist_in.append(at)
@@ -548,7 +554,6 @@ def apply(weights: Mapping[str, torch.Tensor], u: Update, checksums: dict | None
                 hist_in.append(0)
                 sizes.append(0)
     size = _count_slab(L.crx_update_total_changes(u.handle), sizes, numels, slab)
-    fine = False
     if keep:
         fresh = []  # tensors without counts of this slab size
         if sizes.count(size) != len(sizes):
@@ -559,12 +564,11 @@ def apply(weights: Mapping[str, torch.Tensor], u: Update, checksums: dict | None
         # tensors without usable counts: one allocation, sliced per tensor
         fresh = [(i, L.crx_apply_hist_words(targets[i].numel(), size)) for i in fresh]
         if fresh:
-            fine = size < min(_COARSE_SLAB, L.crx_apply_count_slab(1 << 40, 0, slab))
             with _hist_lock:
                 for i, _ in fresh:
                     _hist_drop(id(targets[i]))
-                room = _FINE_COUNTS - _fine if fine else None
-            if fine:
+                room = _FINE_COUNTS - _fine
+            if _fine_slab(slab, size):
                 wanted, fresh = fresh, []
                 for i, w in wanted:
                     if 4 * w <= room:
@@ -608,12 +612,10 @@ def apply(weights: Mapping[str, torch.Tensor], u: Update, checksums: dict | None
             hg = _hist.get
             for a, buf, v in zip(targets, bufs, after):
                 e = hg(id(a))
-                if buf is None:
-                    continue
                 if e is not None and e[2] is buf and e[0]() is a:  # the same counts: a new version only
-                    _hist[id(a)] = (e[0], v, buf, slab, dev, e[5], size, e[7])
-                else:
-                    _hist_store(a, buf, slab, dev, size, fine)
+                    _hist[id(a)] = (e[0], v, buf, slab, dev, e[5], size)
+                elif buf is not None:
+                    _hist_store(a, buf, slab, dev, size)
     if checksums is not None:  # record the version after our own write
         checksums.update({name: (c, v) for name, c, v in zip(names, header_chk, after)})
     return changed.value
