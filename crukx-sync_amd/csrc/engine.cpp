@@ -1373,6 +1373,13 @@ struct PartCheck {
     std::vector<uint64_t> delta, full;
 };
 
+// The decoder runs on the auxiliary stream where the main stream has enough to do beside it: so many weights
+// to stream for their counts (pass A), or, with the counts kept, so many slabs to scan.  Elsewhere the
+// streams' waits for each other cost what they hide.  Measured, apply with the decoder beside pass A and the
+// scans / behind them (us): without kept counts 26M weights 295 / 297, 60M 378 / 394, 134M 539 / 564, 400M
+// 1043 / 1135, 2.4B 4492 / 4562; with them 26M 287 / 283, 60M 355 / 350, 232M (7,100 slabs) 990 / 996, 455M
+// (13,900 slabs) 1251 / 1267, 1.3B (20,400 slabs) 2181 / 2200.
+constexpr uint64_t kForkWeights = 1ULL << 25;
 constexpr uint32_t kForkTiles = 8192;
 
 // One part of an update, or the whole of it (codec.py:578-717): decode, locate, verify, then write.
@@ -1418,12 +1425,13 @@ PartCheck apply_part(const Update &u, const Layout &L, const ApplyPart &P, const
     launch_block_map(d_groups, (uint32_t)G, bmap, binfo, s);
 
     // The decoder needs nothing from the receiver's weights: it runs on the auxiliary stream while
-    // the main stream takes the exponent counts (pass A) and their scans, where those take longer than the
-    // two streams take to wait for each other (30-40 us: kForkTiles).
+    // the main stream takes pass A and the scans, where those are long enough (kForkWeights).
     unsigned long long *dz = ar.get<unsigned long long>(C);
     unsigned long long *blk_sum = ar.get<unsigned long long>(B), *blk_prefix = ar.get<unsigned long long>(B + 1);
     hc.mark("apply_upload");
-    Fork fork(s, tiles > kForkTiles);
+    uint64_t streamed = 0;
+    for (const TensorDesc &d : descs) streamed += d.hist_in ? 0 : d.numel;
+    Fork fork(s, streamed >= kForkWeights || tiles > kForkTiles);
     DecodeArgs da{d_descs, sh.pay, sh.pay_words, sh.bb + P.b0, sh.boff + P.b0, B, d_groups, (uint32_t)G, bmap,
                   sh.lim, sh.off, sh.syms, sh.n_syms, dz, blk_sum, bad, sh.n_tables, sh.bit0,
                   wave_decodes(u, P) ? sh.lens : nullptr};
@@ -1703,7 +1711,8 @@ void apply(const Update &u, const uint8_t *payload_dev, uint16_t *const *targets
         // A small call's tables travel with the part's other uploads (a copy less: 7-10 us).  In a larger one
         // they go ahead, so that the device copies and sums the block table while the host prepares the
         // part (1.5B weights, 1%: together 3% slower than ahead, beside 0.7% between runs).
-        const bool together = small || L.tiles <= kForkTiles;
+        constexpr uint32_t kTogetherTiles = 8192;
+        const bool together = small || L.tiles <= kTogetherTiles;
         if (!together) {
             tb.commit(ar, s);
             uploaded();

@@ -491,8 +491,32 @@ def scenario_kept_counts() -> None:
     print("kept counts: within the limit", flush=True)
 
 
+def scenario_fork() -> None:
+    """The decoder has a stream of its own where the receiver's weights are streamed beside it, from 2^25 of
+    them on: not with counts kept, nor in smaller calls."""
+    import torch
+
+    import crukx_sync
+    import oracle
+    from crukx_sync import _native
+
+    waits = ctypes.c_int.in_dll(_native.lib(), "simt_stream_waits")
+    for n, forks in ((1 << 25, True), ((1 << 25) - 1, False)):
+        a = torch.full((n,), 0x3F80, dtype=torch.int16)
+        b = a.clone()
+        b[::100_003] += 1
+        w, chk = {"w": a.clone()}, {}
+        for upd, to, expect in ((oracle.encode_update({"w": a}, {"w": b}), b, forks),
+                                (oracle.encode_update({"w": b}, {"w": a}), a, False)):
+            waits.value = 0
+            crukx_sync.apply_update(w, upd, chk)
+            assert torch.equal(w["w"], to)
+            assert (waits.value > 0) == expect, (n, waits.value)
+    print("fork: by the weights streamed", flush=True)
+
+
 SCENARIOS = {"parity": scenario_parity, "small4_flips": scenario_small4_flips, "rejected_early": scenario_rejected_early,
-             "group_message": scenario_group_message, "parts": scenario_parts, "long_codes": scenario_long_codes, "kept_counts": scenario_kept_counts,
+             "group_message": scenario_group_message, "parts": scenario_parts, "long_codes": scenario_long_codes, "kept_counts": scenario_kept_counts, "fork": scenario_fork,
              "pinned_exhausted": scenario_pinned_exhausted,
              "device_offsets": scenario_device_offsets}
 

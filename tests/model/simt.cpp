@@ -395,7 +395,12 @@ hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
     *ms = 0.0f;
     return hipSuccess;
 }
-hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+extern "C" int simt_stream_waits;  // streams made to wait for another so far
+int simt_stream_waits = 0;
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) {
+    ++simt_stream_waits;
+    return hipSuccess;
+}
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 // How many more pinned allocations succeed (negative: all), for tests of calls that run out of them.
 extern "C" int simt_host_mallocs_left;

@@ -97,3 +97,7 @@ def test_kept_counts_stay_within_their_limit(model):
     """Tensors applied in calls of their own keep exponent counts of slabs as small as 512 elements, as
     many bytes as their weights: all of a process's together are limited."""
     assert "within the limit" in _run(model, "kept_counts")
+
+
+def test_decoder_beside_the_weights_stream(model):
+    assert "by the weights streamed" in _run(model, "fork")
