@@ -555,6 +555,13 @@ struct UploadBatch {
     T *at(size_t i) const { return reinterpret_cast<T *>(dev + items[i].off); }
 };
 
+// CRX_LARGE_PATHS (any value): calls of every size take what large ones take, the largest slabs, a lane per
+// block, the auxiliary stream, scans in several launches, uploads of their own, for tests of those at sizes
+// an oracle can check.  Read at each call's start; a call runs on one thread.
+thread_local bool t_large = false;
+void read_large_paths() { t_large = std::getenv("CRX_LARGE_PATHS") != nullptr; }
+bool large_paths() { return t_large; }
+
 // The caller's `slab` is the reference's _SLAB (codec.py:30): tensors of more elements get the exact
 // group-size check before decoding (codec.py:598-604); 0 or less means its default, 2^24.
 uint64_t group_check_numel(int32_t slab) { return slab > 0 ? (uint64_t)slab : (1ULL << 24); }
@@ -578,6 +585,7 @@ uint32_t slab_size(int32_t slab) {
 // takes half the slab: the select pass holds a slab's changes in a 2048-entry LDS list and reads longer
 // ones from HBM (1.5B weights at 3% changed, 1966 per slab: select 2.75 ms, 2.39 in slabs of 32768).
 uint32_t slab_for(int32_t slab_req, uint64_t elements, uint64_t changes) {
+    if (large_paths()) return slab_size(slab_req);
     uint32_t s = 512;
     while (s < 32768 && elements > (uint64_t)s * 4096) s *= 2;
     if (elements >= (1ULL << 30) && changes <= elements / 65536 * 1600) s = 65536;
@@ -616,7 +624,7 @@ void finish_layout(Layout &L, uint32_t slab) {
     }
     for (uint32_t t = 0; t < L.descs.size(); ++t) {
         const TensorDesc &d = L.descs[t];
-        if (most <= kScanTensorTiles) {
+        if (most <= kScanTensorTiles && !large_paths()) {
             const uint32_t n = d.n_tiles <= kScanFewTiles ? 256 : kScanFewCols;
             for (uint32_t k = 0; k < 256; k += n) L.cols.push_back(ScanCols{t, k, n, 0});
         } else {
@@ -626,7 +634,7 @@ void finish_layout(Layout &L, uint32_t slab) {
             L.tensor_chunk_begin.push_back((uint32_t)L.chunks.size());
         }
     }
-    if (L.tiles <= kHostTileMap)
+    if (L.tiles <= kHostTileMap && !large_paths())
         for (uint32_t t = 0; t < L.descs.size(); ++t) L.tile_tensor.insert(L.tile_tensor.end(), L.descs[t].n_tiles, t);
 }
 
@@ -1363,7 +1371,7 @@ struct ApplyPart {
 // Whether a part's blocks take a wavefront each or a lane each (a part's own bits are not looked up: the
 // whole payload's bound them).
 bool wave_decodes(const Update &u, const ApplyPart &P) {
-    return P.B <= kDecWaveBlocks && u.payload_len <= kDecWaveBits / 8;
+    return !large_paths() && P.B <= kDecWaveBlocks && u.payload_len <= kDecWaveBits / 8;
 }
 
 // What one part's pass found: error flags, and per tensor of the part the checksum delta and (for
@@ -1431,7 +1439,7 @@ PartCheck apply_part(const Update &u, const Layout &L, const ApplyPart &P, const
     hc.mark("apply_upload");
     uint64_t streamed = 0;
     for (const TensorDesc &d : descs) streamed += d.hist_in ? 0 : d.numel;
-    Fork fork(s, streamed >= kForkWeights || tiles > kForkTiles);
+    Fork fork(s, streamed >= kForkWeights || tiles > kForkTiles || large_paths());
     DecodeArgs da{d_descs, sh.pay, sh.pay_words, sh.bb + P.b0, sh.boff + P.b0, B, d_groups, (uint32_t)G, bmap,
                   sh.lim, sh.off, sh.syms, sh.n_syms, dz, blk_sum, bad, sh.n_tables, sh.bit0,
                   wave_decodes(u, P) ? sh.lens : nullptr};
@@ -1646,7 +1654,7 @@ void apply(const Update &u, const uint8_t *payload_dev, uint16_t *const *targets
     }
     const size_t i_lim = tb.add(lim.data(), lim.size()), i_off = tb.add(off.data(), off.size()),
                  i_syms = tb.add(syms.data(), syms.size()), i_lens = tb.add(lens.data(), lens.size());
-    const bool small = !payload_dev && 4 * B_all + u.payload_len <= kSmallUpdate;
+    const bool small = !large_paths() && !payload_dev && 4 * B_all + u.payload_len <= kSmallUpdate;
     const uint64_t pad_words = (u.payload_len + 7) / 8 + 2;  // a copied payload's words, zero-padded by two
     const size_t i_bb = small ? tb.add(static_cast<const uint8_t *>(u.block_table), 4 * B_all) : 0,
                  i_pay = small ? tb.add_padded(u.payload_host, u.payload_len, 8 * pad_words) : 0;
@@ -1779,6 +1787,7 @@ int32_t guarded(char *err, uint64_t errlen, F &&f) {
         if (err && errlen) std::snprintf(err, (size_t)errlen, "%s", m);
     };
     try {
+        read_large_paths();
         t_stage.abandon();
         f();
         if (g_timing) timing_collect(false);
@@ -1963,6 +1972,7 @@ int32_t crx_apply_counts(const crx_update *u, const uint8_t *payload_dev, uint16
 }
 
 int32_t crx_apply_count_slab(uint64_t elements, uint64_t changes, int32_t slab) {
+    read_large_paths();
     return (int32_t)slab_for(slab, elements, changes);
 }
 

@@ -268,6 +268,7 @@ void launch_block_map(const GroupDev *groups, uint32_t n_groups, uint32_t *bmap,
 // kScanOneMax elements: one workgroup, one launch.
 constexpr uint64_t kScanOneMax = 32768;
 uint64_t scan_parts(uint64_t n);
+bool large_paths();  // engine.cpp: whether this call takes what large ones take, whatever its size
 void launch_scan_u64(const unsigned long long *in, uint64_t n, unsigned long long *out, unsigned long long *part,
                      hipStream_t s);
 void launch_scan_u32(const uint32_t *in, uint64_t n, unsigned long long *out, unsigned long long *part, hipStream_t s);

@@ -2709,7 +2709,7 @@ static void launch_scan(const char *name, const T *in, uint64_t n, unsigned long
         CRX_LAUNCH(name, k_scan_empty, 1, 1, s, out);
         return;
     }
-    if (n <= kScanOneMax) {
+    if (n <= kScanOneMax && !large_paths()) {
         CRX_LAUNCH(name, k_scan_one<T>, 1, kScanOneThreads, s, in, (uint32_t)n, out);
         return;
     }

@@ -226,7 +226,8 @@ def test_small4_every_header_byte_every_block_boundary_and_10k_payload_flips():
 
 
 def test_small4_widened_flips_with_small_slabs(monkeypatch):
-    """The same flips with 16,384-element slabs (every tensor takes the group-size check; many slabs
+    """The same flips with slabs of at most 16,384 elements (8,192 in a call of this size, 16,384 in
+    test_large_paths.py; every tensor takes the group-size check; many slabs
     per tensor), edge values whose exponent-0 changes put slabs across several 64-exponent windows, a
     dense patch whose windows overflow the select pass's LDS list, the receiver's caches warm, and
     2,000 more payload flips inside the blocks of those slabs."""

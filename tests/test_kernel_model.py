@@ -40,8 +40,8 @@ def model():
     return run.build()
 
 
-def _run(lib: str, scenario: str) -> str:
-    r = subprocess.run([sys.executable, os.path.join(HERE, "run.py"), scenario], env=run.env(lib),
+def _run(lib: str, scenario: str, **env) -> str:
+    r = subprocess.run([sys.executable, os.path.join(HERE, "run.py"), scenario], env={**run.env(lib), **env},
                        capture_output=True, text=True, timeout=1500)
     assert r.returncode == 0, (r.stdout[-2000:], r.stderr[-6000:])
     return r.stdout
@@ -101,3 +101,12 @@ def test_kept_counts_stay_within_their_limit(model):
 
 def test_decoder_beside_the_weights_stream(model):
     assert "by the weights streamed" in _run(model, "fork")
+
+
+@pytest.mark.parametrize("scenario,says", [
+    ("parity", "parity "), ("rejected_early", "the receiver unchanged each time"), ("device_offsets", "12 applies exact"),
+    ("parts", "chained applies exact"), ("long_codes", "exact")])
+def test_what_large_calls_take(model, scenario, says):
+    """The scenarios above in slabs as large as _SLAB allows, decoded by a lane per block on a stream of its
+    own, with every scan in several launches: what calls take that are too large for the emulator."""
+    assert says in _run(model, scenario, CRX_LARGE_PATHS="1")

@@ -347,9 +347,10 @@ def test_rejected_update_leaves_the_weights_as_they_were(name):
 
 @pytest.mark.parametrize("rho", [0.005, 0.02, 0.025, 0.1, 0.6, "mixed"])
 def test_change_densities_across_target_list_sizes(rho):
-    """Slabs with a few hundred to tens of thousands of changes (the select pass keeps up to a fixed
-    number of a window's targets in LDS, more for denser updates, and reads larger lists from HBM):
-    exact round trips and the oracle's bytes.  "mixed": one dense slab in a sparse update."""
+    """Slabs with up to half of their elements changed, and, in slabs of 65536 elements
+    (test_large_paths.py), with a few hundred to tens of thousands of changes (the select pass keeps up to
+    a fixed number of a window's targets in LDS, more for denser updates, and reads larger lists from
+    HBM): exact round trips and the oracle's bytes.  "mixed": one dense slab in a sparse update."""
     g = torch.Generator().manual_seed(7 if rho == "mixed" else int(rho * 1000))
     n = 400_003 if rho == "mixed" else 200_003
     a = (torch.randn(n, generator=g) * 0.02).to(torch.bfloat16)
@@ -391,8 +392,8 @@ def test_many_large_residuals_bytes_equal_oracle(n_large):
 
 
 def test_exponent_counts_are_not_reused_across_slab_sizes(monkeypatch):
-    """Counts recorded with one slab size are recomputed, not reused, when the slab size changes
-    between updates of the same receiver tensors (their layout differs)."""
+    """Counts recorded with one _SLAB are recomputed, not reused, when _SLAB changes between updates of the
+    same receiver tensors (their layout differs where it sets the slabs: test_large_paths.py)."""
     g = torch.Generator().manual_seed(9)
     cur = {"a": (torch.randn(200_003, generator=g) * 0.02).to(torch.bfloat16),
            "b": (torch.randn(96, 1024, generator=g) * 0.02).to(torch.bfloat16)}
