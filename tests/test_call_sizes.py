@@ -1,6 +1,8 @@
 """Calls of different sizes take different slab sizes (crx_apply_count_slab) and kernels: results are the
 oracle's at the sizes where the choice changes."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -157,12 +159,13 @@ def test_blocks_of_long_remainders():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("gap", [14, 15, 16, 66, 67, 90])
-def test_workgroups_of_long_bit_strings(gap):
+@pytest.mark.parametrize("gap,extra", [(14, 0), (15, 0), (16, 0), (66, 0), (67, 0), (67, 15), (90, 0)])
+def test_workgroups_of_long_bit_strings(gap, extra):
     """Workgroups of 4096 changes that take gap + 1 bits each (a million changes in one run hold the Rice
-    parameter at 0): as many as are staged at most (16 per change), as are assembled in LDS at most (68),
-    and more."""
-    dense, far = 1 << 20, 3 * 4096 + 17
+    parameter at 0): as many bits as are staged at most (16 per change), more, as many as LDS surely holds
+    (67; its 8704 words hold 68 where the string begins with a word, as after a run of 15 changes more),
+    and as many as it does not."""
+    dense, far = (1 << 20) + extra, 3 * 4096 + 17
     a = torch.full((dense + gap * far,), 0x3F80, dtype=torch.int16)
     b = a.clone()
     b[:dense] += 1
@@ -173,6 +176,8 @@ def test_workgroups_of_long_bit_strings(gap):
     bits = 8 * _native.lib().crx_update_payload_len(crukx_sync.parse(upd).handle)
     # the first of the far changes follows the run at once
     assert 0 <= bits - (2 * dense + 2 + (far - 1) * (gap + 1)) < 8
+    # change 2^20 + 4096, with which a workgroup begins, as the 4096 after it
+    assert ((2 * dense + 2 + (4096 - extra - 1) * (gap + 1)) % 32 == 0) == (extra == 15)
     recv = _cuda(old)
     crukx_sync.apply_update(recv, upd)
     assert torch.equal(recv["w"].cpu(), b)
@@ -234,3 +239,44 @@ def test_a_small_calls_workspace_after_a_large_call_of_as_many_slabs():
     after = peaks(small)
     # without a hint of its own size a call takes its workspace in chunks of 8 MiB, the last not full
     assert all(x <= y + (8 << 20) for x, y in zip(after, alone)), (alone, after)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [513, 20_003, 700_001])
+@pytest.mark.parametrize("slab", [0, 4096])
+def test_apply_entries_of_the_c_interface(n, slab):
+    """crx_apply, crx_apply_cached with counts of the largest slabs that `slab` allows (written, then kept
+    over two updates) and crx_apply_counts with smaller ones: exact, and nothing written when a checksum
+    is not the receiver's."""
+    a, b = scenarios.rl_pair(n, lr=4e-5, seed=n)
+    L, dev = _native.lib(), torch.device("cuda")
+    there, back = (crukx_sync.parse(oracle.encode_update({"w": x}, {"w": y})) for x, y in ((a, b), (b, a)))
+    ups, target = (there, back), a.cuda()
+    err, changed = _native.errbuf(), ctypes.c_uint64()
+
+    def call(entry, u, *args, cached=None):
+        ws = _native.Workspace(target.device)
+        rc = entry(u.handle, None, (ctypes.c_void_p * 1)(target.data_ptr()), (ctypes.c_uint64 * 1)(n),
+                   (ctypes.c_int32 * 1)(cached is not None), (ctypes.c_uint64 * 1)(cached or 0), *args, slab,
+                   _native.stream_of(target.device), ws.fn, None, ctypes.byref(changed), err, 512)
+        ws.check()
+        torch.cuda.synchronize()
+        ws.release()
+        return rc
+
+    def holds(x):
+        return torch.equal(target.cpu().view(torch.int16), x.view(torch.int16))
+
+    def counts(size):
+        buf = torch.full((L.crx_apply_hist_words(n, size),), -1, dtype=torch.int32, device=dev)
+        return buf, (ctypes.c_void_p * 1)(buf.data_ptr())
+
+    assert call(L.crx_apply, ups[0]) == _native.OK and holds(b) and changed.value > 0
+    assert call(L.crx_apply, ups[0]) == _native.CORRUPT and holds(b)
+    assert call(L.crx_apply, ups[1]) == _native.OK and holds(a)
+    for entry, size in ((L.crx_apply_cached, ()), (L.crx_apply_counts, (256,))):
+        buf, p = counts(size[0] if size else slab)  # (held: p is its address)
+        none = (ctypes.c_void_p * 1)()
+        assert call(entry, ups[0], none, p, *size) == _native.OK and holds(b)
+        assert call(entry, ups[1], p, p, *size, cached=oracle.checksum(b)) == _native.OK and holds(a)
+        assert call(entry, ups[0], p, p, *size, cached=oracle.checksum(a) ^ 1) == _native.CORRUPT and holds(a)
