@@ -1609,8 +1609,8 @@ __global__ __launch_bounds__(64) void k_decode_wave(DecodeArgs a) {
         const uint32_t s = (shift + ln) & 31, wl = (shift + ln + 31) >> 5, rs = 32 - s;
         uint64_t runs = 0;  // rows of 64 positions with runs of 32 or more
         for (uint32_t i0 = 0; i0 < n / 64; i0 += 4) {
-            uint32_t len[4], peek[4], fixed[4];
-            bool any = false;
+            uint32_t len[4], peek[4], fixed[4], to[4];
+            bool any = false, far_any = false;
 #pragma unroll
             for (uint32_t u = 0; u < 4; ++u) {
                 const uint32_t *const w = &S.w[wl + 2 * (i0 + u)];
@@ -1619,27 +1619,35 @@ __global__ __launch_bounds__(64) void k_decode_wave(DecodeArgs a) {
                 fixed[u] = q + 1 + rice;
                 peek[u] = (uint32_t)(((((uint64_t)hi << 32) | lo) << min(fixed[u], 63u)) >> 47);
                 len[u] = S.len[peek[u] >> (17 - kPeekBits)];
-                if (q == 32 || fixed[u] > 47) len[u] = 0;
-                any = any || len[u] == 0;
+                const bool past = q == 32 || fixed[u] > 47;  // not all in the window
+                far_any = far_any || past;
+                any = any || past || len[u] == 0;
+                to[u] = 64 * (i0 + u) + ln + fixed[u] + len[u];
             }
             if (ballot(any)) {
 #pragma unroll
                 for (uint32_t u = 0; u < 4; ++u) {
-                    const bool run = fixed[u] == 33 + rice;
-                    if (fixed[u] > 47) {  // the Huffman code lies past the window's first half: one word on
-                        const uint32_t *const w = &S.w[wl + 2 * (i0 + u)];
-                        const uint32_t lo = funnel_right(w[1], w[2], rs), lo2 = funnel_right(w[2], w[3], rs);
-                        peek[u] = (uint32_t)(((((uint64_t)lo << 32) | lo2) << (fixed[u] - 32)) >> 47);
+                    const uint32_t l = len[u] ? len[u] : length_of(peek[u]);
+                    to[u] = l <= 17 ? to[u] - len[u] + l : (uint32_t)kLongCode;
+                }
+                if (ballot(far_any)) {
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; ++u) {
+                        const bool run = fixed[u] == 33 + rice;
+                        if (run) {
+                            to[u] = kRunCode;
+                        } else if (fixed[u] > 47) {  // the Huffman code lies past the window's first half: one word on
+                            const uint32_t *const w = &S.w[wl + 2 * (i0 + u)];
+                            const uint32_t lo = funnel_right(w[1], w[2], rs), lo2 = funnel_right(w[2], w[3], rs);
+                            const uint32_t l = length_of((uint32_t)(((((uint64_t)lo << 32) | lo2) << (fixed[u] - 32)) >> 47));
+                            to[u] = l <= 17 ? 64 * (i0 + u) + ln + fixed[u] + l : (uint32_t)kLongCode;
+                        }
+                        if (ballot(run)) runs |= 1ULL << (i0 + u);
                     }
-                    len[u] = run ? 19u : len[u] ? len[u] : length_of(peek[u]);
-                    if (ballot(run)) runs |= 1ULL << (i0 + u);
                 }
             }
 #pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) {
-                const uint32_t p = 64 * (i0 + u) + ln;
-                S.next[p] = (uint16_t)(len[u] <= 17 ? p + fixed[u] + len[u] : len[u] == 18 ? (uint32_t)kLongCode : (uint32_t)kRunCode);
-            }
+            for (uint32_t u = 0; u < 4; ++u) S.next[64 * (i0 + u) + ln] = (uint16_t)to[u];
         }
         wave_fence();
         while (runs) {  // from the last such row back: the position 32 bits on is known
@@ -1712,17 +1720,17 @@ __global__ __launch_bounds__(64) void k_decode_wave(DecodeArgs a) {
 #pragma unroll
         for (uint32_t u = 0; u < 4; ++u) {
             x[u] = window(shift + S.code[min(done + 64 * u + ln, found - 1)]);
-            q[u] = ~x[u] ? (uint32_t)__builtin_clzll(~x[u]) : 64u;
+            q[u] = (uint32_t)__builtin_clzll(~x[u] | 1);  // 63: that or more
             any = any || q[u] + 1 + rice > 47;
         }
         if (ballot(any)) {  // remainder and code not both in the window: the run's end, then a window of their own
 #pragma unroll
             for (uint32_t u = 0; u < 4; ++u) {
                 const uint32_t p = shift + S.code[min(done + 64 * u + ln, found - 1)];
-                while (q[u] % 64 == 0 && q[u]) {  // every run in the map ends in the segment's words
+                for (bool more = q[u] == 63; more;) {  // every run in the map ends in the segment's words
                     const uint64_t y = ~window(p + q[u]);
                     q[u] += y ? (uint32_t)__builtin_clzll(y) : 64u;
-                    if (y) break;
+                    more = !y;
                 }
                 x[u] = window(p + q[u] + 1);
             }
