@@ -425,19 +425,20 @@ def _apply_inputs(names, numels, weights, checksums):
 
 
 def _count_slab(changes, sizes, numels, slab):
-    """The slab size of an apply of `changes` changes to tensors of `numels` elements, whose usable counts
+    """The slab size of an apply of changes() changes to tensors of `numels` elements, whose usable counts
     have slabs of `sizes` (0: none; empty: no counts are kept): that of the counts that cover half of the
     elements, so that a receiver whose updates hold now more, now fewer of its tensors or changes keeps its
     counts; else the one that suits the update.  Counts of slabs smaller than half of those are not used:
     the call's tables would be as many times as large (a model first applied tensor by tensor, then as a
     whole), and counting again is one read of the weights.  (1.5B weights after an apply of each tensor by
     itself, in the pieces' slabs: 3.6 ms and 1.2 GB of workspace; in its own: 2.5 ms and 0.44 GB.)"""
-    L = _native.lib()
     elements = sum(numels)
-    suits = L.crx_apply_count_slab(elements, changes, slab)
-    if sizes and 2 * sizes[0] >= suits and sizes.count(sizes[0]) == len(sizes):  # the usual: all of one size
-        return sizes[0]
-    by = {}
+    if sizes and sizes.count(sizes[0]) == len(sizes):  # the usual: all of one size
+        # (crx_apply_count_slab gives a call at least 4096 times its slab size unless that is 512, and at
+        # most 65536: half of it is not more than these)
+        if sizes[0] >= _COARSE_SLAB or elements <= 8192 * sizes[0]:
+            return sizes[0]
+    suits, by = _native.lib().crx_apply_count_slab(elements, changes(), slab), {}
     for size, k in zip(sizes, numels):
         if 2 * size >= suits:
             by[size] = by.get(size, 0) + k
@@ -553,7 +554,7 @@ def apply(weights: Mapping[str, torch.Tensor], u: Update, checksums: dict | None
                 bufs.append(None)
                 hist_in.append(0)
                 sizes.append(0)
-    size = _count_slab(L.crx_update_total_changes(u.handle), sizes, numels, slab)
+    size = _count_slab(lambda: L.crx_update_total_changes(u.handle), sizes, numels, slab)
     if keep:
         fresh = []  # tensors without counts of this slab size
         if sizes.count(size) != len(sizes):

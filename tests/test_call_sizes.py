@@ -38,14 +38,28 @@ def test_count_slab_of_a_whole_model_applied_in_pieces_before(n, kept, want):
     L, pieces = _native.lib(), 7_600_000_000 // n
     changes = 76_000_000
     assert L.crx_apply_count_slab(n, n // 100, 1 << 24) == kept
-    assert codec._count_slab(changes, [kept] * pieces, [n] * pieces, 1 << 24) == want
-    assert codec._count_slab(changes, [kept, 65536] * (pieces // 2), [n] * (pieces // 2 * 2), 1 << 24) == (want if 2 * kept >= want else 65536)
-    assert codec._count_slab(changes, [], [n] * pieces, 1 << 24) == 65536
-    assert codec._count_slab(n // 100, [want], [n], 1 << 24) == want
-    assert codec._count_slab(n // 100, [kept], [n], 1 << 24) == kept
+    assert codec._count_slab(lambda: changes, [kept] * pieces, [n] * pieces, 1 << 24) == want
+    assert codec._count_slab(lambda: changes, [kept, 65536] * (pieces // 2), [n] * (pieces // 2 * 2), 1 << 24) == (want if 2 * kept >= want else 65536)
+    assert codec._count_slab(lambda: changes, [], [n] * pieces, 1 << 24) == 65536
+    assert codec._count_slab(lambda: n // 100, [want], [n], 1 << 24) == want
+    assert codec._count_slab(lambda: n // 100, [kept], [n], 1 << 24) == kept
     # the same tensors at a few more changes or elements than the rule's lines: their counts are used
-    assert codec._count_slab(changes * 3, [65536] * pieces, [n] * pieces, 1 << 24) == 65536
-    assert codec._count_slab(changes, [32768] * pieces, [n] * pieces, 1 << 24) == 32768
+    assert codec._count_slab(lambda: changes * 3, [65536] * pieces, [n] * pieces, 1 << 24) == 65536
+    assert codec._count_slab(lambda: changes, [32768] * pieces, [n] * pieces, 1 << 24) == 32768
+
+
+def test_count_slab_of_counts_of_one_size():
+    """Counts of one size (that some call takes) are used when it is at least half of what suits the call,
+    at every call size."""
+    f = _native.lib().crx_apply_count_slab
+    calls = [e for k in range(8, 34) for e in ((1 << k) - 1, 1 << k, (1 << k) + 1)]
+    for slab in (0, 128, 600, 1000, 4096, 40_000, 1 << 24):
+        for size in {f(e, 0, slab) for e in calls}:
+            for elements in calls:
+                for changes in (0, elements // 30):
+                    suits = f(elements, changes, slab)
+                    got = codec._count_slab(lambda: changes, [size], [elements], slab)
+                    assert got == (size if 2 * size >= suits else suits), (elements, slab, changes, size)
 
 
 @pytest.mark.gpu
