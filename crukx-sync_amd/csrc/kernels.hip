@@ -1589,6 +1589,7 @@ __global__ __launch_bounds__(64) void k_decode_wave(DecodeArgs a) {
             }
             ++done;
             rel += q + 1 + len;
+            wave_fence();
         };
         if (far) {
             const uint64_t q = unary_run(a, at, end, qmax);
@@ -1705,7 +1706,6 @@ __global__ __launch_bounds__(64) void k_decode_wave(DecodeArgs a) {
         far = found < done + 8;
         if (!pos) {  // the first code passes the segment
             read_one(unary_run(a, at, end, qmax));
-            wave_fence();
             continue;
         }
         // the codes found (the last one again past them), from the payload in LDS; all loads together
