@@ -557,7 +557,7 @@ struct UploadBatch {
 
 // CRX_LARGE_PATHS (any value): calls of every size take what large ones take, the largest slabs, a lane per
 // block, the auxiliary stream, scans in several launches, uploads of their own, for tests of those at sizes
-// an oracle can check.  Read at each call's start; a call runs on one thread.
+// an oracle can check.  Read at the start of encode and apply, each of which runs on one thread.
 thread_local bool t_large = false;
 void read_large_paths() { t_large = std::getenv("CRX_LARGE_PATHS") != nullptr; }
 bool large_paths() { return t_large; }
@@ -1179,6 +1179,7 @@ void encode_parts(const Layout &L, uint64_t limit, uint32_t slab, const int32_t 
 void encode(int32_t n, const uint16_t *const *olds, const uint16_t *const *news, const uint64_t *numels,
             const int32_t *has_cache, const uint64_t *cache_vals, int32_t slab_req, hipStream_t s, Arena &ar,
             crx_encoded &E) {
+    read_large_paths();
     uint64_t elements = 0;
     for (int32_t t = 0; t < n; ++t) elements += numels[t];
     const uint32_t slab = slab_for(slab_req, elements, 0);
@@ -1559,6 +1560,7 @@ void apply(const Update &u, const uint8_t *payload_dev, uint16_t *const *targets
     *changed = 0;
     const uint32_t T = (uint32_t)u.tensors.size();
     if (!T) return;
+    read_large_paths();
     HostClock hc;
     const uint64_t C = u.total_changes;
     Layout L;
@@ -1787,7 +1789,6 @@ int32_t guarded(char *err, uint64_t errlen, F &&f) {
         if (err && errlen) std::snprintf(err, (size_t)errlen, "%s", m);
     };
     try {
-        read_large_paths();
         t_stage.abandon();
         f();
         if (g_timing) timing_collect(false);
